@@ -66,6 +66,7 @@ struct Tuning
     double csr_order = 1.0;             // CSR features: visit large inputs' rows in spatial order
     double heap_tail = 1.0;             // search heaps: nodes past 20 in global memory (k > 21); 2: per wave slot always
     double staging = 0.0;               // LDS staging of cell rows: 0 never, 1 radius + budgeted kNN at k >= 32, 2 always
+    double wave_k_max = 108.0;          // kNN up to this k: one wave per query (0: never), else a lane per query
     double fuse_multiscale = 0.0;       // radius + multiscale: features in the search kernel (1) or a CSR kernel after it (0)
 };
 Tuning g_tune;
@@ -92,6 +93,7 @@ const KnobName kKnobs[] = {
     {"csr_order", &Tuning::csr_order},
     {"heap_tail", &Tuning::heap_tail},
     {"staging", &Tuning::staging},
+    {"wave_k_max", &Tuning::wave_k_max},
     {"fuse_multiscale", &Tuning::fuse_multiscale},
 };
 
@@ -622,6 +624,15 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
     }
 }
 
+// Whether a kNN search takes the wave-per-query kernel: up to k = 108, the
+// largest rows it keeps.  Faster than a lane per query with a heap at every
+// size and k measured (us per call, before -> now: 257 queries on 1,000
+// points at k = 10 228 -> 100; 10 k points at k = 20 227 -> 135; 100 k LiDAR
+// points at k = 20 1061 -> 430; 10 M 11.25 -> 7.9 ms; 4 M at k = 50
+// 13.2 -> 4.3 ms; 1 M at k = 100 7.1 -> 2.1 ms).  Past 108 a row no longer
+// fits the lanes that sort it and the general search is the only one.
+bool wave_path(uint32_t k) { return k <= kWaveMaxK && (double)k <= tuning().wave_k_max; }
+
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,
 // when query != data, sort the queries into level 0.  kNN sizes h_0 from the
 // target occupancy (k used for sizing); radius searches use one level with
@@ -641,7 +652,11 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
     p.is_radius = is_radius ? 1 : 0;
     p.cap = cap;
     p.max_levels = is_radius ? 1 : std::max(1, std::min(kMaxLevels, (int)t.grid_levels));
-    p.knn_occupancy = t.knn_occupancy;
+    // the wave-per-query search keeps the regions of 3D clouds in registers
+    // with slightly smaller cells (1 M uniform points at k = 50: 877 us
+    // per call with 0.35 k points per cell, 874 with 0.28 k, 1.24 ms with
+    // 0.2 k; 4 M LiDAR points 4.4, 4.2 and 4.3 ms)
+    p.knn_occupancy = t.knn_occupancy * (!is_radius && wave_path(k) ? 0.85 : 1.0);
     p.knn_cell_points_max = t.knn_cell_points_max;
     p.radius_cell_factor = t.radius_cell_factor;
     p.level_ratio = t.grid_level_ratio;
@@ -721,7 +736,30 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     a.gheap_keys = w.gheap_keys;
     a.heap_tail = tail_layout(hp, m);
     a.tail_pairs = hp.tail_pairs;
-    if (mode == kModeKnn || mode == kModeKnnFeat)
+    if ((mode == kModeKnn || mode == kModeKnnFeat) && wave_path(k))
+    {
+        WaveArgs b{};
+        b.tab = w.tab;
+        b.data = data;
+        b.queries = qs;
+        b.n_query = m;
+        b.k = k;
+        // A region of 27 cells on a surface is 9 k / (pi c) balls of the k-th
+        // distance for c points in it: with 4 k of them nearly every query
+        // is closed by its region and few go on to scan the ball (10 M
+        // LiDAR points, k = 20: 1.6 k 8.2 ms per step, 2.5 k 8.0, 4 k 7.9;
+        // 4 M at k = 50: 1.6 k 4.5-5.3, 2.5 k and 4 k 4.2).
+        b.need = 4 * k;
+        // up to 64 queries per wave (those of a cell share its candidates),
+        // fewer where that would leave the chip short of waves
+        b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, m / 8192));
+        b.margin = a.margin;
+        b.out_idx = (uint32_t*)out_idx;
+        b.out_d2 = out_d2;
+        b.out_feat = out_feat;
+        HIP_TRY(launch_wave_knn(mode, b, s));
+    }
+    else if (mode == kModeKnn || mode == kModeKnnFeat)
     {
         // Budgeted passes, finest level first: a query whose k-th neighbour
         // lies beyond +-2 cells of the level is flagged and, compacted and in
@@ -1595,11 +1633,14 @@ int pgeof_autotune(const char* workload, const float* xyz, int64_t n, uint32_t k
     std::vector<Tuning> cand{base};
     if (family == kFamKnn)
     {
+        // (the wave-per-query search has no heaps and stages no rows)
+        const bool wave = k <= kWaveMaxK && (double)k <= base.wave_k_max;
         for (double cpp : {4.0, 8.0, 16.0})
             for (double occ : {0.25, 0.35, 0.5})
                 for (double lds : {65536.0, 32768.0})
                     for (double st : {0.0, 2.0})
                     {
+                        if (wave && (lds != 65536.0 || st != 0.0)) continue;
                         Tuning t = base;
                         t.grid_cells_per_point = cpp;
                         t.knn_occupancy = occ;

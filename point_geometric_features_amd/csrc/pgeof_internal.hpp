@@ -119,6 +119,23 @@ struct SearchArgs
     uint32_t n_scales;
 };
 
+// Arguments of the wave-per-query kNN kernel.
+struct WaveArgs
+{
+    const LevelTable* tab;
+    const float* data;      // the caller's points (fused features gather from it)
+    const float4* queries;  // sorted queries (x, y, z, bits of original query index)
+    uint32_t n_query;
+    uint32_t k;
+    uint32_t need;          // points the region of a query's level should hold (>= k)
+    uint32_t q_per_wave;    // consecutive queries per wave, 1..64
+    float margin;           // slack of the cell faces, relative to h
+    uint32_t* out_idx;      // (n_query, k), rows = original query index
+    float* out_d2;          // (n_query, k) or nullptr
+    float* out_feat;        // (n_query, 11), fused features
+};
+constexpr uint32_t kWaveMaxK = 108;  // largest k of the wave-per-query kernel (128 kept candidates per query)
+
 // Simple linear device arena carved out of one allocation.  Every region
 // starts on a 256-byte boundary of the address space, not only of the
 // offset: regions hold 64-bit atomics and 16-byte vectors, and the base of an
@@ -173,6 +190,7 @@ hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const uint32_t* c
                                  hipStream_t s);
 hipError_t launch_search(int mode, const SearchArgs& a, int block, size_t lds_bytes, bool global_heap, bool budget,
                          hipStream_t s);
+hipError_t launch_wave_knn(int mode, const WaveArgs& a, hipStream_t s);  // pgeof_wave.hip
 // reorder queries (and their bounds) by bound, largest first; count needs
 // 2049 entries, key and rank n_max
 hipError_t launch_order_by_bound(const float4* q, const float* bound, uint32_t n_max, const uint64_t* n_dev,

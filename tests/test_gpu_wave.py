@@ -1,0 +1,147 @@
+"""kNN with one wave per query against the lane-per-query search and the oracle.
+
+The wave kernel serves k <= 108; wave_k_max = 0 sends the same call to the
+general path, which must give the same indices and squared distances bit for
+bit, and the fused features the bits of compute_features on that CSR.
+"""
+import numpy as np
+import pytest
+import torch
+
+import point_geometric_features_amd as pgeof
+from oracle import oracle as O
+from point_geometric_features_amd import capi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+class _Knobs:
+    def __init__(self, **kw):
+        self.kw = kw
+
+    def __enter__(self):
+        self.old = {k: capi.get_tuning(k) for k in self.kw}
+        for k, v in self.kw.items():
+            capi.set_tuning(k, v)
+
+    def __exit__(self, *exc):
+        for k, v in self.old.items():
+            capi.set_tuning(k, v)
+
+
+def _both(data, query, k, **knobs):
+    with _Knobs(**knobs):
+        gi, gd = pgeof.knn_search(data, query, k)
+    with _Knobs(wave_k_max=0):
+        ri, rd = pgeof.knn_search(data, query, k)
+    np.testing.assert_array_equal(gi, ri)
+    np.testing.assert_array_equal(gd, rd)
+    return gi, gd
+
+
+def _fused(xyz, k):
+    x = torch.from_numpy(xyz).cuda()
+    nn = torch.empty(len(xyz) * k, dtype=torch.int32, device="cuda")
+    ptr = torch.empty(len(xyz) + 1, dtype=torch.int32, device="cuda")
+    f = torch.empty((len(xyz), 11), dtype=torch.float32, device="cuda")
+    d = torch.empty(len(xyz) * k, dtype=torch.float32, device="cuda")
+    capi.knn_features_device(x, k, nn, ptr, f, sqr_dist=d)
+    torch.cuda.synchronize()
+    return nn.cpu().numpy().view(np.uint32).reshape(-1, k), d.cpu().numpy().reshape(-1, k), f.cpu().numpy()
+
+
+# row classes of the kernel end at 12, 27, 54 and 108 (109: the general path)
+@pytest.mark.parametrize("k", [1, 11, 12, 13, 16, 27, 28, 32, 48, 54, 55, 64, 65, 96, 108, 109])
+@pytest.mark.parametrize("scene", ["lidar", "cube"])
+def test_row_classes(scene, k):
+    xyz = scenes.lidar_scene(40_003, seed=k, extent=18.0) if scene == "lidar" else scenes.uniform_cube(40_003, seed=k)
+    gi, gd = _both(xyz, xyz, k)
+    rows = np.random.default_rng(k).choice(len(xyz), 500, replace=False)
+    oi, od = O.knn(xyz, xyz[rows], k, kdtree=True)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+    fi, fd, f = _fused(xyz, k)
+    np.testing.assert_array_equal(fi, gi)
+    np.testing.assert_array_equal(fd, gd)
+    nn, ptr = scenes.knn_csr(gi)
+    np.testing.assert_array_equal(f, pgeof.compute_features(xyz, nn, ptr))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 257, 1000])
+def test_small_clouds(n):
+    xyz = scenes.uniform_cube(n, seed=n)
+    for k in sorted({1, min(n, 5), min(n, 64), min(n, 100)}):
+        gi, gd = _both(xyz, xyz, k)
+        oi, od = O.knn(xyz, xyz, k, kdtree=False)
+        np.testing.assert_array_equal(gi, oi)
+        np.testing.assert_array_equal(gd, od)
+
+
+def _clouds():
+    rng = np.random.default_rng(5)
+    lattice = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), -1).reshape(-1, 3).astype(np.float32)
+    dense = rng.normal(0, 0.05, size=(20_000, 3))
+    far = rng.uniform(-50, 50, size=(300, 3))
+    line = np.zeros((5000, 3))
+    line[:, 0] = rng.uniform(0, 100, 5000)
+    return {
+        "lattice": np.concatenate([lattice, lattice[::-1] * np.float32(2)]),
+        "one_point": np.full((3000, 3), 7.25, np.float32),
+        "few_values": rng.integers(0, 3, size=(6000, 3)).astype(np.float32),
+        "outliers": np.concatenate([dense, far]).astype(np.float32),
+        "one_far": np.concatenate([rng.normal(0, 0.1, size=(4000, 3)), [[900.0, -700.0, 300.0]]]).astype(np.float32),
+        "line": line.astype(np.float32),
+        "plane_far": (np.c_[rng.uniform(0, 30, (15_000, 2)), np.zeros(15_000)] + [1e5, 1e5, 0]).astype(np.float32),
+        "spike": np.concatenate([rng.uniform(0, 1, (9000, 3)), 0.5 + 1e-4 * rng.normal(size=(9000, 3))]).astype(np.float32),
+    }
+
+
+@pytest.mark.parametrize("name", ["lattice", "one_point", "few_values", "outliers", "one_far", "line", "plane_far",
+                                  "spike"])
+@pytest.mark.parametrize("k", [9, 20, 50, 100])
+def test_shapes(name, k):
+    """Ties at the k-th place, duplicates, isolated points (cubes that grow),
+    regions too full for the registers, flat and far clouds."""
+    xyz = np.ascontiguousarray(_clouds()[name])
+    gi, gd = _both(xyz, xyz, k)
+    rows = np.random.default_rng(k).choice(len(xyz), 300, replace=False)
+    rows[-1] = len(xyz) - 1
+    oi, od = O.knn(xyz, xyz[rows], k, kdtree=False)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+
+
+@pytest.mark.parametrize("k", [5, 20, 40, 80])
+def test_queries_off_the_data(k):
+    rng = np.random.default_rng(k)
+    data = scenes.lidar_scene(30_001, seed=k, extent=15.0)
+    q = rng.uniform(-200, 220, size=(3001, 3)).astype(np.float32)
+    q[::2] = rng.uniform(-1, 16, size=(1501, 3)).astype(np.float32)
+    q[7] = [np.nan, 0, 0]
+    q[8] = [0, np.inf, 0]
+    gi, gd = _both(data, q, k)
+    assert (gi[7] == 0xFFFFFFFF).all() and np.isinf(gd[8]).all()
+    ok = np.setdiff1d(np.arange(len(q)), [7, 8])
+    oi, od = O.knn(data, q[ok], k, kdtree=False)
+    np.testing.assert_array_equal(gi[ok], oi)
+    np.testing.assert_array_equal(gd[ok], od)
+
+
+def test_data_that_is_not_finite():
+    xyz = scenes.uniform_cube(3000, seed=3)
+    xyz[10] = [np.nan, 0.5, 0.5]
+    xyz[20] = [np.inf, 0.5, 0.5]
+    q = scenes.uniform_cube(300, seed=4)
+    _both(xyz, q, 20)
+    small = xyz[:30].copy()  # rows that need the points without a finite distance
+    _both(small, q, 28)
+
+
+@pytest.mark.parametrize("knobs", [{"grid_levels": 1}, {"grid_levels": 4}, {"grid_levels": 3, "grid_level_ratio": 4},
+                                   {"knn_occupancy": 0.05, "grid_cells_per_point": 32}, {"knn_occupancy": 3.0},
+                                   {"grid_cells_per_point": 1, "grid_levels": 1}],
+                         ids=lambda d: ",".join(f"{k}={v}" for k, v in d.items()))
+@pytest.mark.parametrize("k", [20, 60])
+def test_grids(knobs, k):
+    xyz = scenes.lidar_scene(50_000, seed=29, extent=20.0)
+    _both(xyz, xyz, k, **knobs)
