@@ -624,12 +624,14 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
     }
 }
 
-// Whether a kNN search takes the wave-per-query kernel: up to k = 108, the
-// largest rows it keeps.  Faster than a lane per query with a heap at every
+// Whether a search takes the wave-per-query kernel: up to k (or cap) = 108,
+// the largest rows it keeps.  Faster than a lane per query with a heap at every
 // size and k measured (us per call, before -> now: 257 queries on 1,000
 // points at k = 10 228 -> 100; 10 k points at k = 20 227 -> 135; 100 k LiDAR
 // points at k = 20 1061 -> 430; 10 M 11.25 -> 7.9 ms; 4 M at k = 50
-// 13.2 -> 4.3 ms; 1 M at k = 100 7.1 -> 2.1 ms).  Past 108 a row no longer
+// 13.2 -> 4.3 ms; 1 M at k = 100 7.1 -> 2.1 ms; radius r = 0.5, at most 64,
+// with features of 2 M points 6.9 -> 3.8 ms; r = 0.2, at most 30, 1 M sparse
+// points 384 -> 268 us).  Past 108 a row no longer
 // fits the lanes that sort it and the general search is the only one.
 bool wave_path(uint32_t k) { return k <= kWaveMaxK && (double)k <= tuning().wave_k_max; }
 
@@ -641,7 +643,7 @@ bool wave_path(uint32_t k) { return k <= kWaveMaxK && (double)k <= tuning().wave
 // the kernels take their grid from the level table and the launches are
 // sized for the largest grid the workspace allows.
 int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, uint32_t k, float radius, bool is_radius,
-               SearchWs& w, SearchArgs& sa, const float4** qs_out, hipStream_t s)
+               bool wave, SearchWs& w, SearchArgs& sa, const float4** qs_out, hipStream_t s)
 {
     const Tuning t = tuning();
     const uint64_t cap = grid_cap(n);
@@ -650,13 +652,17 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
     p.k = k;
     p.radius = radius;
     p.is_radius = is_radius ? 1 : 0;
+    p.wave = wave ? 1 : 0;
     p.cap = cap;
-    p.max_levels = is_radius ? 1 : std::max(1, std::min(kMaxLevels, (int)t.grid_levels));
+    // radius searches: one level, or for the wave-per-query search a second one
+    // with half its cells' edge for the dense parts (2 M LiDAR points, r = 0.5,
+    // at most 64, features included: one level 5.9 ms per call, two 3.8, three 3.8)
+    p.max_levels = std::max(1, std::min(is_radius ? (wave ? 2 : 1) : kMaxLevels, (int)t.grid_levels));
     // the wave-per-query search keeps the regions of 3D clouds in registers
     // with slightly smaller cells (1 M uniform points at k = 50: 877 us
     // per call with 0.35 k points per cell, 874 with 0.28 k, 1.24 ms with
     // 0.2 k; 4 M LiDAR points 4.4, 4.2 and 4.3 ms)
-    p.knn_occupancy = t.knn_occupancy * (!is_radius && wave_path(k) ? 0.85 : 1.0);
+    p.knn_occupancy = t.knn_occupancy * (wave ? 0.85 : 1.0);
     p.knn_cell_points_max = t.knn_cell_points_max;
     p.radius_cell_factor = t.radius_cell_factor;
     p.level_ratio = t.grid_level_ratio;
@@ -714,7 +720,8 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     a.n_scales = n_scales;
     const float4* qs = nullptr;
     const bool is_radius = mode == kModeRadius || mode == kModeRadiusCsr || mode == kModeRadiusMulti;
-    int rc = build_grid(data, n, query, m, k, radius, is_radius, w, a, &qs, s);
+    const bool wave = mode != kModeRadiusMulti && wave_path(k);
+    int rc = build_grid(data, n, query, m, k, radius, is_radius, wave, w, a, &qs, s);
     if (rc) return rc;
     a.data = data;
     a.queries = qs;
@@ -736,7 +743,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     a.gheap_keys = w.gheap_keys;
     a.heap_tail = tail_layout(hp, m);
     a.tail_pairs = hp.tail_pairs;
-    if ((mode == kModeKnn || mode == kModeKnnFeat) && wave_path(k))
+    if (wave)
     {
         WaveArgs b{};
         b.tab = w.tab;
@@ -754,10 +761,18 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         // fewer where that would leave the chip short of waves
         b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, m / 8192));
         b.margin = a.margin;
-        b.out_idx = (uint32_t*)out_idx;
+        if (is_radius)
+        {
+            uint32_t bits;
+            std::memcpy(&bits, &a.r2, 4);
+            b.limit = bits ? std::min(bits - 1u, 0x7FC00000u) : 0xFFFFFFFFu;
+            b.r2 = a.r2;
+            b.out_count = a.out_count;
+        }
+        b.out_idx = (uint32_t*)a.out_idx;
         b.out_d2 = out_d2;
         b.out_feat = out_feat;
-        HIP_TRY(launch_wave_knn(mode, b, s));
+        HIP_TRY(launch_wave_search(mode, b, s));
     }
     else if (mode == kModeKnn || mode == kModeKnnFeat)
     {
@@ -1003,7 +1018,7 @@ int selected_host(const T* xyz, int64_t n, T search_radius, uint32_t max_knn, co
     if (wa.off > wa.size) return fail(PGEOF_ENOMEM, "workspace too small");
     SearchArgs sa{};
     const float4* qs = nullptr;
-    rc = build_grid(d_xf, (uint32_t)n, d_xf, (uint32_t)n, cap, (float)search_radius, true, w, sa, &qs, s);
+    rc = build_grid(d_xf, (uint32_t)n, d_xf, (uint32_t)n, cap, (float)search_radius, true, false, w, sa, &qs, s);
     if (rc) return rc;
     // this host entry point synchronises anyway: the kernel takes level 0 by value
     LevelTable tab;

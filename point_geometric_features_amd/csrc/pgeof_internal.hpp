@@ -76,6 +76,7 @@ struct PlanArgs
     uint32_t k;  // kNN: k (sizes the cells); radius: unused
     float radius;
     int is_radius;
+    int wave;        // radius: levels for the wave-per-query search
     uint64_t cap;  // largest G of level 0 (grid_cells_per_point * n)
     int max_levels;
     double knn_occupancy, knn_cell_points_max, radius_cell_factor, level_ratio;
@@ -119,7 +120,7 @@ struct SearchArgs
     uint32_t n_scales;
 };
 
-// Arguments of the wave-per-query kNN kernel.
+// Arguments of the wave-per-query search kernel.
 struct WaveArgs
 {
     const LevelTable* tab;
@@ -130,11 +131,14 @@ struct WaveArgs
     uint32_t need;          // points the region of a query's level should hold (>= k)
     uint32_t q_per_wave;    // consecutive queries per wave, 1..64
     float margin;           // slack of the cell faces, relative to h
+    uint32_t limit;         // radius: largest float bits of a hit's squared distance, 0xFFFFFFFF: none can be one
+    float r2;               // radius: search_radius * search_radius
     uint32_t* out_idx;      // (n_query, k), rows = original query index
     float* out_d2;          // (n_query, k) or nullptr
     float* out_feat;        // (n_query, 11), fused features
+    uint32_t* out_count;    // radius: hits per original query (at most k) or nullptr
 };
-constexpr uint32_t kWaveMaxK = 108;  // largest k of the wave-per-query kernel (128 kept candidates per query)
+constexpr uint32_t kWaveMaxK = 108;  // largest k of that kernel (128 kept candidates per query)
 
 // Simple linear device arena carved out of one allocation.  Every region
 // starts on a 256-byte boundary of the address space, not only of the
@@ -190,7 +194,7 @@ hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const uint32_t* c
                                  hipStream_t s);
 hipError_t launch_search(int mode, const SearchArgs& a, int block, size_t lds_bytes, bool global_heap, bool budget,
                          hipStream_t s);
-hipError_t launch_wave_knn(int mode, const WaveArgs& a, hipStream_t s);  // pgeof_wave.hip
+hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s);  // pgeof_wave.hip
 // reorder queries (and their bounds) by bound, largest first; count needs
 // 2049 entries, key and rank n_max
 hipError_t launch_order_by_bound(const float4* q, const float* bound, uint32_t n_max, const uint64_t* n_dev,

@@ -390,6 +390,7 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
     double ext[3], emax;
     plan_extent(bb, ext, emax);
     const double hcap = tab->hcap;
+    int levels = p.is_radius ? 1 : p.max_levels;
     double h;
     if (!(emax > 0.0))
         h = 1.0;
@@ -397,6 +398,17 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
     {
         const double r = fabs((double)p.radius);
         h = isfinite(r) && r > 0.0 ? r * p.radius_cell_factor : emax;
+        if (p.wave && isfinite(r) && r > 0.0)
+        {
+            // the coarsest level's cells span the radius (a little more, for
+            // the float region tests), so that 3x3x3 of them hold the ball;
+            // finer levels, halving, as far as the cap allows serve the
+            // dense parts
+            h = fmax(2.0 * p.radius_cell_factor * (r * 1.0005 + 2e-6 * emax), hcap);
+            int finer = 0;
+            while (finer + 1 < p.max_levels && 0.5 * h >= hcap) h *= 0.5, ++finer;
+            levels = finer + 1;
+        }
         h = fmax(h, hcap);
     }
     else
@@ -410,9 +422,9 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         if (m1 > T) h = h1 * sqrt(T / m1);
         h = fmax(h, hcap);
     }
-    const double ratio = fmax(2.0, fmin(8.0, p.level_ratio));
+    const double ratio = p.is_radius ? 2.0 : fmax(2.0, fmin(8.0, p.level_ratio));
     int nl = 0;
-    for (int l = 0; l < p.max_levels; ++l)
+    for (int l = 0; l < levels; ++l)
     {
         Level L;
         uint64_t G;

@@ -1,4 +1,5 @@
-// kNN search with one wavefront per query, for gfx950 (k <= kWaveMaxK).
+// kNN and radius search with one wavefront per query, for gfx950 (k or cap <=
+// kWaveMaxK; a radius search is a kNN search of its cap with a limit).
 //
 // A wave takes up to 64 consecutive queries of the cell-sorted order, one at
 // a time.  The 3x3x3 cells around a query's cell, on the finest pyramid level
@@ -9,9 +10,9 @@
 // kept candidates go to LDS; when 64 / G queries are collected, G lanes sort
 // the row of each in registers and the wave writes the rows.  A query whose
 // threshold reaches past its region scans the cells of that ball; one whose
-// region holds too few points (or too many for the registers) first finds the
-// cells nearest to it that hold k.  The fused mode ends with the features,
-// one query per lane.
+// region holds too few points (or too many for the registers) scans balls that
+// grow until they hold k.  The fused mode ends with the features, one query
+// per lane.
 //
 // What bounds it: instruction issue and the latency of the few dependent
 // loads per region, at 13 waves per CU (LDS rows) and 12 (k > 27, registers):
@@ -210,14 +211,16 @@ struct Candidates
     // the squared distance on a surface), then by bisection of the bits.
     // Thresholds up to `closed` are preferred (no point outside the scanned
     // cells is nearer); past it open = true, and `outer` bounds all distances
-    // that are expected.  Ties at the k-th distance may leave no such
-    // threshold: then n > most, and ties() bounds the indices.
+    // that are expected.  No threshold passes `limit` (a radius search's):
+    // with fewer than k candidates up to it tau = limit and n < k.  Ties at
+    // the k-th distance may leave no threshold: then n > most, and ties()
+    // bounds the indices.
     __device__ __forceinline__ uint32_t select(uint32_t k, uint32_t most, uint32_t guess, uint32_t closed,
-                                               uint32_t outer, uint32_t& n, bool& open) const
+                                               uint32_t outer, uint32_t limit, uint32_t& n, bool& open) const
     {
         const float target = 0.5f * (float)(k + most);
         int lo = -1, hi = 0;
-        uint32_t clo = 0, chi = 0, cap = closed;
+        uint32_t clo = 0, chi = 0, cap = min(closed, limit);
         bool hi_known = false;
         open = false;
         uint32_t tau = min(guess, cap);
@@ -227,7 +230,16 @@ struct Candidates
             if (c < k)
             {
                 lo = (int)tau, clo = c;
-                if (tau == cap) cap = cap < outer ? outer : kNanBits, open = true;
+                if (tau == cap)
+                {
+                    if (cap == limit)
+                    {
+                        n = c;
+                        return tau;
+                    }
+                    cap = cap < outer ? min(outer, limit) : limit;
+                    open = true;
+                }
             }
             else
             {
@@ -330,7 +342,6 @@ template <int G>
 constexpr uint32_t kGroupsOf = G <= 2 ? 8 : 12;
 // Streamed candidates collected in LDS before the farthest are dropped.
 constexpr uint32_t kBufGroups = 6, kBufKeys = 64 * kBufGroups;
-constexpr int kNearCells = 16;  // edge of the largest box taken from the last query's threshold
 constexpr uint32_t kAhead = 3;  // groups of 64 of them loaded together
 
 // Block b's place in the sorted order of the queries.  Runs of kRun blocks go
@@ -367,14 +378,16 @@ __device__ __forceinline__ uint32_t work_block(uint32_t b, uint32_t nb)
 
 // G: lanes that sort one query's row of kPerLane * G kept candidates
 template <int MODE, int G>
-__global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
+__global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
 {
+    constexpr bool RADIUS = MODE == kModeRadius || MODE == kModeRadiusCsr;
     constexpr uint32_t kGroups = kGroupsOf<G>;
     constexpr uint32_t kMost = (uint32_t)(kPerLane * G);  // candidates kept per query
     constexpr uint32_t kBatch = 64 / G;                   // queries collected before their rows are sorted
     constexpr uint32_t kStride = kMost + 1;               // odd: the rows start on different LDS banks
-    __shared__ uint64_t kept[kBatch * kStride];
-    __shared__ uint64_t buf[kBufKeys];
+    __shared__ uint64_t lds[kBatch * kStride + kBufKeys];
+    uint64_t* const kept = lds;
+    uint64_t* const buf = lds + kBatch * kStride;
     const uint32_t lane = threadIdx.x;
     const uint32_t k = a.k;
 
@@ -397,7 +410,9 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
     // region's faces, changes no result.
     float4 qv = make_float4(0.f, 0.f, 0.f, 0.f);
     if (lane < nq) qv = a.queries[t0 + lane];
-    const uint64_t finite = __ballot(isfinite(qv.x) && isfinite(qv.y) && isfinite(qv.z));
+    uint64_t finite = __ballot(isfinite(qv.x) && isfinite(qv.y) && isfinite(qv.z));
+    if (RADIUS && a.limit == 0xFFFFFFFFu) finite = 0;  // no distance is below the radius
+    const uint32_t limit = RADIUS ? a.limit : kNanBits;
     const PGEOF_CONST Level* L0 = scalar_level(a.tab, 0);
     const float relx = (float)((double)qv.x - L0->lo[0]), rely = (float)((double)qv.y - L0->lo[1]),
                 relz = (float)((double)qv.z - L0->lo[2]);
@@ -409,23 +424,125 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
         return (int)fminf(fmaxf(rel * ih, 0.0f), (float)(g - 1));
     };
 
+    // How far the 3x3x3 cells around cell (c0, c1, c2) of a level cover this
+    // lane's query: distance bits up to which a ball around it stays inside
+    // them (faces on the grid's border do not count), and bits no distance to
+    // a point in them exceeds.
+    auto cover = [&](int c0, int c1, int c2, float h, int a0, int a1, int a2, uint32_t& inner, uint32_t& all) {
+        const float xl = relx - (float)(c0 - 1) * h, xh = (float)(c0 + 2) * h - relx;
+        const float yl = rely - (float)(c1 - 1) * h, yh = (float)(c1 + 2) * h - rely;
+        const float zl = relz - (float)(c2 - 1) * h, zh = (float)(c2 + 2) * h - relz;
+        float g = INFINITY;
+        g = c0 > 1 ? fminf(g, xl) : g;
+        g = c0 < a0 - 2 ? fminf(g, xh) : g;
+        g = c1 > 1 ? fminf(g, yl) : g;
+        g = c1 < a1 - 2 ? fminf(g, yh) : g;
+        g = c2 > 1 ? fminf(g, zl) : g;
+        g = c2 < a2 - 2 ? fminf(g, zh) : g;
+        const float gm = fmaxf(g - h * a.margin - slack, 0.0f);
+        inner = g == INFINITY ? kNanBits : __float_as_uint(gm * gm * 0.99996f);
+        const float ex = fmaxf(xl, xh), ey = fmaxf(yl, yh), ez = fmaxf(zl, zh);
+        all = __float_as_uint((ex * ex + ey * ey + ez * ez) * 1.001f);
+    };
+
+    // Sorted rows of the queries first .. first + count, `stride` keys apart
+    // in LDS; lane s holds the number of keys of query first + s.
+    auto write_rows = [&](uint32_t first, uint32_t count, uint32_t stride, uint32_t keys) {
+        for (uint32_t s = 0; s < count; ++s)
+        {
+            const uint32_t qorig = readlane(__float_as_uint(qv.w), first + s);
+            uint32_t* oi = a.out_idx + (size_t)qorig * k;
+            float* od = a.out_d2 ? a.out_d2 + (size_t)qorig * k : nullptr;
+            const uint32_t hits = RADIUS ? min(readlane(keys, s), k) : k;
+#pragma unroll
+            for (uint32_t e0 = 0; e0 < kMost; e0 += 64)
+            {
+                const uint32_t e = e0 + lane;
+                if (e >= (MODE == kModeRadiusCsr ? hits : k)) continue;
+                const uint64_t key = lds[s * stride + min(e, stride - 1u)];
+                const bool none = RADIUS ? e >= hits : key == kNoKey;
+                oi[e] = none ? 0xFFFFFFFFu : (uint32_t)key;
+                // past the hits 0, and r^2 in the last slot (nanoflann's
+                // RKNNResultSet::init)
+                const float pad = !RADIUS ? INFINITY : (e == k - 1 ? a.r2 : 0.0f);
+                if (od) od[e] = none ? pad : __uint_as_float((uint32_t)(key >> 32));
+            }
+        }
+        if (RADIUS && a.out_count)
+        {
+            // lane s counts the hits of query first + s
+            const uint32_t qorig = from_lane(__float_as_uint(qv.w), (first + lane) & 63u);
+            if (lane < count) a.out_count[qorig] = min(keys, k);
+        }
+    };
+
+    if constexpr (RADIUS)
+    {
+        // A wave whose queries have at most 16 points around them each:
+        // one query per lane, its region's points one after the other (1 M
+        // uniform points with their own point in the ball: a wave per query
+        // would spend its instructions on one candidate).
+        const PGEOF_CONST Level* L = scalar_level(a.tab, nl - 1);
+        const float h = (float)L->h, ih = (float)L->inv_h;
+        const int a0 = L->g[0], a1 = L->g[1], a2 = L->g[2];
+        const uint32_t* __restrict__ tcs = L->cs;
+        const float4* __restrict__ pts = L->pts;
+        const int cx = cell32(relx, ih, a0), cy = cell32(rely, ih, a1), cz = cell32(relz, ih, a2);
+        const bool mine = (finite >> lane) & 1ull;
+        uint32_t st[9], end[9], around = 0;
+#pragma unroll
+        for (int r = 0; r < 9; ++r)
+        {
+            const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+            st[r] = end[r] = 0;
+            if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
+            {
+                const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
+                st[r] = gload(tcs, at + (uint32_t)max(cx - 1, 0));
+                end[r] = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 9; ++r) around += end[r] - st[r];
+        uint32_t inner, all;
+        cover(cx, cy, cz, h, a0, a1, a2, inner, all);
+        if (__ballot(mine && (around > (uint32_t)kPerLane || inner < limit)) == 0)
+        {
+            constexpr uint32_t kSparse = (uint32_t)kPerLane + 1;
+            static_assert(64 * kSparse <= sizeof(lds) / 8, "rows of the sparse case");
+            uint64_t* row = lds + lane * kSparse;
+            uint32_t n = 0;
+#pragma unroll
+            for (int r = 0; r < 9; ++r)
+                for (uint32_t j = st[r]; j < end[r]; ++j)
+                {
+                    const float4 p = gload(pts, j);
+                    const uint32_t d = min(__float_as_uint(sqdist32(qv.x, qv.y, qv.z, p.x, p.y, p.z)), kNanBits);
+                    if (d <= limit) row[n++] = ((uint64_t)d << 32) | __float_as_uint(p.w);
+                }
+            double v[kPerLane];
+#pragma unroll
+            for (int r = 0; r < kPerLane; ++r) v[r] = __longlong_as_double((long long)((uint32_t)r < n ? row[r] : kNoKey));
+            sort_rows<1>(v, lane);
+#pragma unroll
+            for (int r = 0; r < kPerLane; ++r) row[r] = (uint64_t)__double_as_longlong(v[r]);
+            wave_sync();
+            write_rows(0, nq, kSparse, n);
+            return;
+        }
+    }
+
     // the current region: the 3x3x3 cells around one of level rl
     uint64_t served = 0;  // queries in that cell
     uint32_t rl = 0;
     int rx = 0, ry = 0, rz = 0;  // the cell
     uint32_t total = 0;          // candidates in the region
     bool in_regs = false;
-    // this lane's query: distance bits up to which a ball around it stays
-    // inside the region (faces on the grid's border do not count), and bits
-    // no distance to a point of the region exceeds
-    uint32_t closed = 0, outer = 0;
+    uint32_t closed = 0, outer = 0;  // how far it covers this lane's query
     float px[kGroups], py[kGroups], pz[kGroups];
     uint32_t pi[kGroups];
 #pragma unroll
     for (uint32_t u = 0; u < kGroups; ++u) px[u] = py[u] = pz[u] = 0.f, pi[u] = 0;
-    // the last query and the threshold that kept at least k candidates of it
-    float lx = 0.f, ly = 0.f, lz = 0.f;
-    uint32_t ltau = kNanBits;
     uint32_t guess = 0;  // distance bits expected to keep about `target` candidates
     const float target = 0.5f * (float)(k + kMost);
 
@@ -475,7 +592,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                 if (total > 64u * kGroups && prev >= k) --rl, total = prev;
                 const uint32_t gl = 16u * rl;
                 rx = readlane(cx, gl), ry = readlane(cy, gl), rz = readlane(cz, gl);
-                in_regs = total >= k && total <= 64u * kGroups;
+                in_regs = (RADIUS || total >= k) && total <= 64u * kGroups;
                 const PGEOF_CONST Level* L = scalar_level(a.tab, rl);
                 if (in_regs)
                 {
@@ -506,21 +623,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                 served = __ballot(cell32(relx, ih, a0) == rx && cell32(rely, ih, a1) == ry &&
                                   cell32(relz, ih, a2) == rz) |
                          (1ull << i);
-                const float xl = relx - (float)(rx - 1) * h, xh = (float)(rx + 2) * h - relx;
-                const float yl = rely - (float)(ry - 1) * h, yh = (float)(ry + 2) * h - rely;
-                const float zl = relz - (float)(rz - 1) * h, zh = (float)(rz + 2) * h - relz;
-                float g = INFINITY;
-                g = rx > 1 ? fminf(g, xl) : g;
-                g = rx < a0 - 2 ? fminf(g, xh) : g;
-                g = ry > 1 ? fminf(g, yl) : g;
-                g = ry < a1 - 2 ? fminf(g, yh) : g;
-                g = rz > 1 ? fminf(g, zl) : g;
-                g = rz < a2 - 2 ? fminf(g, zh) : g;
-                const float gm = fmaxf(g - h * a.margin - slack, 0.0f);
-                closed = g == INFINITY ? kNanBits : __float_as_uint(gm * gm * 0.99996f);
-                const float ex = fmaxf(xl, xh), ey = fmaxf(yl, yh), ez = fmaxf(zl, zh);
-                outer = __float_as_uint((ex * ex + ey * ey + ez * ez) * 1.001f);
-
+                cover(rx, ry, rz, h, a0, a1, a2, closed, outer);
                 const uint64_t later = finite & ~served & (~0ull << i);
                 if (later) look_up((uint32_t)__ffsll((unsigned long long)later) - 1u);
             }
@@ -535,7 +638,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                 {
                     // an even spread over the region's area
                     const float h = (float)scalar_level(a.tab, rl)->h;
-                    guess = uniform(__float_as_uint(h * h * 2.8f * target / (float)total));
+                    guess = uniform(__float_as_uint(h * h * 2.8f * target / (float)max(total, 1u)));
                 }
                 auto search = [&](auto groups) {
                     constexpr int NG = decltype(groups)::value;
@@ -547,7 +650,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                         c.id[u] = pi[u];
                     }
                     bool open;
-                    tau = c.select(k, kMost, guess, readlane(closed, i), readlane(outer, i), n, open);
+                    tau = c.select(k, kMost, guess, readlane(closed, i), readlane(outer, i), limit, n, open);
                     bounded = tau < 0x7F800000u;
                     done = bounded && !open;
                     if (done) n = c.store(row, k, kMost, tau, n);
@@ -570,10 +673,10 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
             if (!done)
             {
                 // ---- the cells of the level that meet the ball of tau.  With
-                // fewer than k candidates at hand (or too many for the
-                // registers) tau first comes from the cells nearest to the
-                // query that hold k points, out of a cube grown until it
-                // does. ----
+                // no threshold at hand (fewer than k candidates, or too many
+                // for the registers) it is taken from the last query's, or an
+                // even spread over the region, and grows until the ball holds
+                // k points: then it holds the k nearest ones. ----
                 const PGEOF_CONST Level* L = scalar_level(a.tab, rl);
                 const double lo0 = L->lo[0], lo1 = L->lo[1], lo2 = L->lo[2], h = L->h, ih = L->inv_h;
                 const int a0 = L->g[0], a1 = L->g[1], a2 = L->g[2];
@@ -581,7 +684,20 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                 const float4* __restrict__ pts = L->pts;
                 const double margin = h * (double)a.margin;
                 const double qx = qxf, qy = qyf, qz = qzf;
-                if (!bounded) tau = kNanBits;
+                double away = 0.0;  // of the query from the grid's box
+                if (!bounded)
+                {
+                    const double dx = fmax(fmax(lo0 - qx, qx - (lo0 + (double)a0 * h)), 0.0),
+                                 dy = fmax(fmax(lo1 - qy, qy - (lo1 + (double)a1 * h)), 0.0),
+                                 dz = fmax(fmax(lo2 - qz, qz - (lo2 + (double)a2 * h)), 0.0);
+                    away = sqrt(dx * dx + dy * dy + dz * dz);
+                    const double w = guess > 0 && guess < 0x7F800000u
+                                         ? 1.25 * (double)__uint_as_float(guess)
+                                         : h * h * 2.8 * (double)target / (double)max(total, 1u);
+                    const double r = fmax(sqrt(w), away + 0.25 * h);
+                    const uint32_t t = uniform(__float_as_uint((float)(r * r)));
+                    tau = min(t < 0x7F800000u ? t : kNanBits, limit);
+                }
                 Box B{0, 0, 0, 0, 0, 0};
                 uint32_t ny = 1, nr = 1;
                 double lim = INFINITY;  // squared distance of the rows of interest
@@ -595,91 +711,17 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                     st = gload(ucs, at + (uint32_t)xa);
                     len = gload(ucs, at + (uint32_t)xb + 1u) - st;
                 };
-                auto set_box = [&](double ext) {
+                for (;;)
+                {
+                    const float w = __uint_as_float(tau);
+                    lim = w < INFINITY ? (double)w * 1.00001 + 1e-37 : INFINITY;
+                    const double ext = sqrt(lim) + margin;
                     B = Box{cell_coord(qx - ext, lo0, ih, a0), cell_coord(qx + ext, lo0, ih, a0),
                             cell_coord(qy - ext, lo1, ih, a1), cell_coord(qy + ext, lo1, ih, a1),
                             cell_coord(qz - ext, lo2, ih, a2), cell_coord(qz + ext, lo2, ih, a2)};
                     B.y0 = (int)uniform((uint32_t)B.y0), B.y1 = (int)uniform((uint32_t)B.y1);
                     B.z0 = (int)uniform((uint32_t)B.z0), B.z1 = (int)uniform((uint32_t)B.z1);
                     ny = (uint32_t)(B.y1 - B.y0 + 1), nr = ny * (uint32_t)(B.z1 - B.z0 + 1);
-                };
-                bool ball = bounded;
-                // k points lie within the last query's threshold of it, so
-                // within that distance plus the way to it of this query
-                bool near_last = false;
-                if (!ball && ltau < 0x7F800000u)
-                {
-                    const double dx = qx - lx, dy = qy - ly, dz = qz - lz;
-                    set_box((sqrt(dx * dx + dy * dy + dz * dz) + sqrt((double)__uint_as_float(ltau))) * 1.0001 + margin);
-                    near_last = (int)uniform((uint32_t)max(B.x1 - B.x0, max(B.y1 - B.y0, B.z1 - B.z0))) < kNearCells;
-                }
-                for (int half = total < k ? 2 : 1; !ball; half += (half + 1) / 2)
-                {
-                    if (!near_last)
-                    {
-                        B = Box{max(rx - half, 0), min(rx + half, a0 - 1), max(ry - half, 0), min(ry + half, a1 - 1),
-                                max(rz - half, 0), min(rz + half, a2 - 1)};
-                        ny = (uint32_t)(B.y1 - B.y0 + 1), nr = ny * (uint32_t)(B.z1 - B.z0 + 1);
-                    }
-                    near_last = false;
-                    // radius around the query whose cells hold k points of
-                    // the box, in 64ths of its farthest corner's distance:
-                    // the rows' inner, middle and whole x ranges counted by
-                    // their far ends
-                    const int xc = min(max(rx, B.x0), B.x1), in = (B.x1 - B.x0) / 8, mid = (B.x1 - B.x0) / 4;
-                    auto reach = [&](double v, double lo, int c0, int c1) {
-                        return fmax(fabs(v - (lo + (double)c0 * h)), fabs(lo + (double)(c1 + 1) * h - v));
-                    };
-                    const double fx = reach(qx, lo0, B.x0, B.x1), fy = reach(qy, lo1, B.y0, B.y1),
-                                 fz = reach(qz, lo2, B.z0, B.z1);
-                    const double step = sqrt(fx * fx + fy * fy + fz * fz) * (1.0001 / 63.0);
-                    uint32_t* bins = reinterpret_cast<uint32_t*>(buf);
-                    wave_sync();
-                    bins[lane] = 0;
-                    wave_sync();
-                    for (uint32_t r0 = 0; r0 < nr; r0 += 64)
-                    {
-                        const uint32_t r = r0 + lane;
-                        if (r < nr)
-                        {
-                            int y, z;
-                            const double g2 = row_gap2(r, y, z);
-                            uint32_t before = 0;
-#pragma unroll
-                            for (int v = 0; v < 3; ++v)
-                            {
-                                const int xa = v == 2 ? B.x0 : max(xc - (v ? mid : in), B.x0);
-                                const int xb = v == 2 ? B.x1 : min(xc + (v ? mid : in), B.x1);
-                                uint32_t st, len;
-                                row_range(y, z, xa, xb, st, len);
-                                const double f = reach(qx, lo0, xa, xb);
-                                const uint32_t bin = min((uint32_t)(sqrt(g2 + f * f) / step), 63u);
-                                if (len > before) atomicAdd(&bins[bin], len - before);
-                                before = len;
-                            }
-                        }
-                    }
-                    wave_sync();
-                    const uint64_t enough = __ballot(wave_scan(bins[lane]) >= k);
-                    wave_sync();
-                    if (enough == 0 && half < max(a0, max(a1, a2))) continue;
-                    lim = INFINITY;
-                    if (enough)
-                    {
-                        const double rad = step * (double)__ffsll((unsigned long long)enough);
-                        lim = rad * rad * 1.00001 + 1e-37;
-                    }
-                    break;
-                }
-                wave_sync();
-                for (;;)
-                {
-                    if (ball)
-                    {
-                        const float w = __uint_as_float(tau);
-                        lim = w < INFINITY ? (double)w * 1.00001 + 1e-37 : INFINITY;
-                        set_box(sqrt(lim) + margin);
-                    }
                     uint32_t n_buf = 0;
                     // the nearest of the collected keys stay (at least k, at
                     // most kMost of them), tau drops to their threshold
@@ -696,7 +738,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                         bool open;
                         uint32_t m;
                         const float t = __uint_as_float(tau) * target * __builtin_amdgcn_rcpf((float)n_buf);
-                        tau = c.select(k, kMost, uniform(__float_as_uint(t)), kNanBits, kNanBits, m, open);
+                        tau = c.select(k, kMost, uniform(__float_as_uint(t)), kNanBits, kNanBits, kNanBits, m, open);
                         n_buf = c.store(buf, k, kMost, tau, m);
                     };
                     // one row of cells per lane, then the rows' points as one
@@ -747,10 +789,15 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
                             if (n_buf > kBufKeys - 64u * kAhead) reduce();
                         }
                     }
-                    if (n_buf > kMost || (!ball && n_buf >= k)) reduce();
+                    if (n_buf > kMost) reduce();
                     n = n_buf;
-                    if (ball) break;
-                    ball = true;
+                    if (n >= k || tau >= limit) break;
+                    // the next ball: the part of the radius past the grid's
+                    // box grows, by the points found (about with its square)
+                    const double f = n ? sqrt(fmin(fmax(1.2 * (double)target / (double)n, 1.5), 8.0)) : 2.8;
+                    const double past = fmax(sqrt((double)w) - away, 0.25 * h) * f + away;
+                    const uint32_t t = uniform(__float_as_uint((float)(past * past)));
+                    tau = min(t < 0x7F800000u ? max(t, tau + 1u) : kNanBits, limit);
                 }
                 wave_sync();
                 for (uint32_t e = lane; e < n; e += 64) row[e] = buf[e];
@@ -758,7 +805,6 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
             }
             guess = uniform(__float_as_uint(__uint_as_float(tau) * target * __builtin_amdgcn_rcpf((float)n)));
             n_kept = lane == s ? n : n_kept;
-            lx = qxf, ly = qyf, lz = qzf, ltau = tau;
         }
 
         // ---- the batch's rows, sorted and written ----
@@ -776,24 +822,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_knn(WaveArgs a)
             for (int r = 0; r < kPerLane; ++r) row[r] = (uint64_t)__double_as_longlong(v[r]);
         }
         wave_sync();
-        for (uint32_t s = 0; s < nb; ++s)
-        {
-            const uint32_t qorig = readlane(__float_as_uint(qv.w), base + s);
-            uint32_t* oi = a.out_idx + (size_t)qorig * k;
-            float* od = a.out_d2 ? a.out_d2 + (size_t)qorig * k : nullptr;
-#pragma unroll
-            for (uint32_t e0 = 0; e0 < kMost; e0 += 64)
-            {
-                const uint32_t e = e0 + lane;
-                if (e < k)
-                {
-                    const uint64_t key = kept[s * kStride + e];
-                    const bool none = key == kNoKey;
-                    oi[e] = none ? 0xFFFFFFFFu : (uint32_t)key;
-                    if (od) od[e] = none ? INFINITY : __uint_as_float((uint32_t)(key >> 32));
-                }
-            }
-        }
+        write_rows(base, nb, kStride, n_kept);
         wave_sync();
     }
 
@@ -851,20 +880,26 @@ template <int G>
 hipError_t launch_wave_g(int mode, const WaveArgs& a, hipStream_t s)
 {
     const uint32_t nb = (a.n_query + a.q_per_wave - 1) / a.q_per_wave;
-    if (mode == kModeKnnFeat)
-        k_wave_knn<kModeKnnFeat, G><<<nb, 64, 0, s>>>(a);
-    else
-        k_wave_knn<kModeKnn, G><<<nb, 64, 0, s>>>(a);
+    switch (mode)
+    {
+        case kModeKnn: k_wave_search<kModeKnn, G><<<nb, 64, 0, s>>>(a); break;
+        case kModeKnnFeat: k_wave_search<kModeKnnFeat, G><<<nb, 64, 0, s>>>(a); break;
+        case kModeRadius: k_wave_search<kModeRadius, G><<<nb, 64, 0, s>>>(a); break;
+        case kModeRadiusCsr: k_wave_search<kModeRadiusCsr, G><<<nb, 64, 0, s>>>(a); break;
+        default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_wave_knn(int mode, const WaveArgs& a, hipStream_t s)
+hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s)
 {
+    static const char* names[4] = {"knn_search", "radius_search", "knn_features_fused", "radius_search_csr"};
     if (a.n_query == 0) return hipSuccess;
-    if (a.k < 1 || a.k > kWaveMaxK || a.q_per_wave < 1 || a.q_per_wave > 64) return hipErrorInvalidValue;
-    ProfScope ps(mode == kModeKnnFeat ? "knn_features_fused" : "knn_search", s);
+    if (mode < 0 || mode > 3 || a.k < 1 || a.k > kWaveMaxK || a.q_per_wave < 1 || a.q_per_wave > 64)
+        return hipErrorInvalidValue;
+    ProfScope ps(names[mode], s);
     // rows of up to 16 G kept candidates, at least about a fifth more than k:
     // a narrower margin takes more steps to find a threshold
     if (a.k <= 12) return launch_wave_g<1>(mode, a, s);

@@ -145,3 +145,87 @@ def test_data_that_is_not_finite():
 def test_grids(knobs, k):
     xyz = scenes.lidar_scene(50_000, seed=29, extent=20.0)
     _both(xyz, xyz, k, **knobs)
+
+
+# ------------------------------------------------------------------ radius ----
+def _radius_both(data, query, r, cap, **knobs):
+    with _Knobs(**knobs):
+        gi, gd = pgeof.radius_search(data, query, r, cap)
+    with _Knobs(wave_k_max=0):
+        ri, rd = pgeof.radius_search(data, query, r, cap)
+    np.testing.assert_array_equal(gi, ri)
+    np.testing.assert_array_equal(gd, rd)
+    return gi, gd
+
+
+# from a point or none in the ball (a query per lane) to more than the cap
+@pytest.mark.parametrize("r", [0.01, 0.05, 0.15, 0.4, 1.5])
+@pytest.mark.parametrize("cap", [1, 12, 13, 30, 54, 64, 108, 109])
+def test_radius(r, cap):
+    xyz = scenes.lidar_scene(30_001, seed=cap, extent=15.0)
+    gi, gd = _radius_both(xyz, xyz, r, cap)
+    rows = np.random.default_rng(cap).choice(len(xyz), 300, replace=False)
+    oi, od, _ = O.radius(xyz, xyz[rows], r, cap, kdtree=True)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+
+
+@pytest.mark.parametrize("name", ["lattice", "one_point", "few_values", "outliers", "one_far", "plane_far", "spike"])
+@pytest.mark.parametrize("r,cap", [(1.0, 20), (0.3, 60), (2.0, 100)])
+def test_radius_shapes(name, r, cap):
+    xyz = np.ascontiguousarray(_clouds()[name])
+    _radius_both(xyz, xyz, r, cap)
+
+
+@pytest.mark.parametrize("r", [0.0, 1e-30, np.inf, -0.5])
+def test_radius_values(r):
+    xyz = scenes.uniform_cube(2000, seed=8)
+    xyz[1] = xyz[0]
+    xyz[5] = [np.nan, 0, 0]
+    q = np.concatenate([xyz, scenes.uniform_cube(100, seed=9) * np.float32(5) - np.float32(2)])
+    q[11] = [np.inf, 0, 0]
+    _radius_both(xyz, np.ascontiguousarray(q), r, 40)
+
+
+def test_radius_queries_off_the_data():
+    rng = np.random.default_rng(3)
+    data = scenes.lidar_scene(20_001, seed=2, extent=12.0)
+    q = rng.uniform(-30, 50, size=(3001, 3)).astype(np.float32)
+    q[::2] = rng.uniform(-1, 13, size=(1501, 3)).astype(np.float32)
+    for r in (0.3, 8.0):
+        _radius_both(data, q, r, 50)
+
+
+@pytest.mark.parametrize("knobs", [{"grid_levels": 1}, {"grid_levels": 2}, {"radius_cell_factor": 0.2},
+                                   {"radius_cell_factor": 1.5}, {"grid_cells_per_point": 1}],
+                         ids=lambda d: ",".join(f"{k}={v}" for k, v in d.items()))
+def test_radius_grids(knobs):
+    xyz = scenes.lidar_scene(50_000, seed=29, extent=20.0)
+    _radius_both(xyz, xyz, 0.35, 50, **knobs)
+
+
+@pytest.mark.parametrize("r", [0.05, 0.5])
+def test_radius_csr(r):
+    xyz = scenes.lidar_scene(60_000, seed=6, extent=25.0)
+    x = torch.from_numpy(xyz).cuda()
+    out = []
+    for kmax in (108, 0):
+        with _Knobs(wave_k_max=kmax):
+            nn = torch.zeros(len(xyz) * 64, dtype=torch.int32, device="cuda")
+            ptr = torch.empty(len(xyz) + 1, dtype=torch.int32, device="cuda")
+            nnz = capi.radius_csr_device(x, r, 64, nn, ptr)
+            out.append((nnz, nn.cpu().numpy(), ptr.cpu().numpy()))
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+    np.testing.assert_array_equal(out[0][2], out[1][2])
+
+
+def test_queries_far_from_a_large_cloud():
+    """Balls that grow from far outside the grid must not take the whole cloud
+    at once (they would hold every point of it)."""
+    data = scenes.lidar_scene(300_000, seed=5, extent=60.0)
+    q = np.random.default_rng(1).uniform(-3000, 3000, size=(200, 3)).astype(np.float32)
+    gi, gd = _both(data, q, 16)
+    oi, od = O.knn(data, q, 16, kdtree=True)
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gd, od)
