@@ -633,7 +633,13 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
 // with features of 2 M points 6.9 -> 3.8 ms; r = 0.2, at most 30, 1 M sparse
 // points 384 -> 268 us).  Past 108 a row no longer
 // fits the lanes that sort it and the general search is the only one.
-bool wave_path(uint32_t k) { return k <= kWaveMaxK && (double)k <= tuning().wave_k_max; }
+// Radius searches of at most 16 stay with it: heaps that small live in
+// registers (1 M LiDAR points, r = 0.37, 50 in the ball: 0.70 ms against 0.81
+// for 16, but 1.34 against 0.82 for 30).
+bool wave_path(uint32_t k, bool radius)
+{
+    return k <= kWaveMaxK && (double)k <= tuning().wave_k_max && !(radius && k <= 16);
+}
 
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,
 // when query != data, sort the queries into level 0.  kNN sizes h_0 from the
@@ -658,11 +664,15 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
     // with half its cells' edge for the dense parts (2 M LiDAR points, r = 0.5,
     // at most 64, features included: one level 5.9 ms per call, two 3.8, three 3.8)
     p.max_levels = std::max(1, std::min(is_radius ? (wave ? 2 : 1) : kMaxLevels, (int)t.grid_levels));
-    // the wave-per-query search keeps the regions of 3D clouds in registers
-    // with slightly smaller cells (1 M uniform points at k = 50: 877 us
-    // per call with 0.35 k points per cell, 874 with 0.28 k, 1.24 ms with
-    // 0.2 k; 4 M LiDAR points 4.4, 4.2 and 4.3 ms)
-    p.knn_occupancy = t.knn_occupancy * (wave ? 0.85 : 1.0);
+    // Points per cell for the wave-per-query search: larger cells share a
+    // region between more queries, up to what keeps the 27 cells of a 3D
+    // cloud's region in registers (6 groups of 64 candidates up to k = 27, 12
+    // above).  1 M uniform points: k = 8 1.07 ms with 0.3 k points per cell,
+    // 0.72 with 0.6 k; k = 20 0.84, 0.77; k = 50 0.87 with 0.3 k, 1.24 with
+    // 0.2 k.  (The knob's default, 0.35, scales to these.)
+    p.knn_occupancy = t.knn_occupancy;
+    if (wave && !is_radius && k)
+        p.knn_occupancy *= (k <= 27 ? std::min(12.0, std::max(5.0, 0.6 * k)) : 0.3 * k) / (0.35 * k);
     p.knn_cell_points_max = t.knn_cell_points_max;
     p.radius_cell_factor = t.radius_cell_factor;
     p.level_ratio = t.grid_level_ratio;
@@ -720,7 +730,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     a.n_scales = n_scales;
     const float4* qs = nullptr;
     const bool is_radius = mode == kModeRadius || mode == kModeRadiusCsr || mode == kModeRadiusMulti;
-    const bool wave = mode != kModeRadiusMulti && wave_path(k);
+    const bool wave = mode != kModeRadiusMulti && wave_path(k, is_radius);
     int rc = build_grid(data, n, query, m, k, radius, is_radius, wave, w, a, &qs, s);
     if (rc) return rc;
     a.data = data;
@@ -757,9 +767,16 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         // LiDAR points, k = 20: 1.6 k 8.2 ms per step, 2.5 k 8.0, 4 k 7.9;
         // 4 M at k = 50: 1.6 k 4.5-5.3, 2.5 k and 4 k 4.2).
         b.need = 4 * k;
-        // up to 64 queries per wave (those of a cell share its candidates),
-        // fewer where that would leave the chip short of waves
-        b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, m / 8192));
+        // Queries per wave: 64 share the candidates of their cells best (10 M
+        // LiDAR points, k = 20: 7.4 ms per call, 32 per wave 8.0); below 2 M
+        // queries shorter waves end more evenly (1 M, k = 10: 0.92 ms with
+        // 32, 1.03 with 64; k = 100 with features 3.0 and 3.2), and small
+        // calls need at least 2048 waves (10 k at k = 20: 122 us with 4 per
+        // wave, 145 with 1).  For radius searches a power of two: the waves
+        // of 64 queries share them where they are sparse.
+        b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, std::max(std::min<uint32_t>(32u, m / 2048), m / 32768)));
+        if (is_radius)
+            while (b.q_per_wave & (b.q_per_wave - 1)) b.q_per_wave &= b.q_per_wave - 1;
         b.margin = a.margin;
         if (is_radius)
         {

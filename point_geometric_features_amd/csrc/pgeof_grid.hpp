@@ -77,4 +77,19 @@ __device__ __forceinline__ Box cube_box(int cx, int cy, int cz, int n, const Lev
                min(cz + n, G.g[2] - 1)};
 }
 
+// t-th element (t in [0, hi - lo]) of the order c, c-1, c+1, c-2, c+2, ...
+// over [lo, hi] with c in [lo, hi]: alternating while both sides last, then
+// the longer side outwards
+__device__ __forceinline__ int nth_near(int t, int c, int lo, int hi)
+{
+    const int below = c - lo, above = hi - c, m = min(below, above);
+    if (t <= 2 * m)
+    {
+        const int d = (t + 1) >> 1;
+        return (t & 1) ? c - d : c + d;
+    }
+    const int r = t - m;
+    return below > above ? c - r : c + r;
+}
+
 }  // namespace pgeof_amd

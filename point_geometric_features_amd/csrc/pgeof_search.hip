@@ -391,6 +391,7 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
     plan_extent(bb, ext, emax);
     const double hcap = tab->hcap;
     int levels = p.is_radius ? 1 : p.max_levels;
+    double ratio = fmax(2.0, fmin(8.0, p.level_ratio));
     double h;
     if (!(emax > 0.0))
         h = 1.0;
@@ -402,12 +403,14 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         {
             // the coarsest level's cells span the radius (a little more, for
             // the float region tests), so that 3x3x3 of them hold the ball;
-            // finer levels, halving, as far as the cap allows serve the
-            // dense parts
-            h = fmax(2.0 * p.radius_cell_factor * (r * 1.0005 + 2e-6 * emax), hcap);
-            int finer = 0;
-            while (finer + 1 < p.max_levels && 0.5 * h >= hcap) h *= 0.5, ++finer;
-            levels = finer + 1;
+            // one of half their edge, or as fine as the cap allows, serves
+            // the dense parts
+            const double top = fmax(2.0 * p.radius_cell_factor * (r * 1.0005 + 2e-6 * emax), hcap);
+            const double fine = fmax(0.5 * top, hcap);
+            const bool two = p.max_levels > 1 && fine < 0.69 * top;
+            h = two ? fine : top;
+            ratio = two ? top / fine : 2.0;
+            levels = two ? 2 : 1;
         }
         h = fmax(h, hcap);
     }
@@ -422,7 +425,6 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         if (m1 > T) h = h1 * sqrt(T / m1);
         h = fmax(h, hcap);
     }
-    const double ratio = p.is_radius ? 2.0 : fmax(2.0, fmin(8.0, p.level_ratio));
     int nl = 0;
     for (int l = 0; l < levels; ++l)
     {
@@ -1013,21 +1015,6 @@ __device__ __forceinline__ int near_index(int i, int c, int lo, int hi)
     c = min(c, hi);
     const int d = (i + 1) >> 1;
     return (i & 1) ? c - d : c + d;
-}
-
-// t-th element (t in [0, hi - lo]) of the order c, c-1, c+1, c-2, c+2, ...
-// over [lo, hi] with c in [lo, hi]: alternating while both sides last, then
-// the longer side outwards
-__device__ __forceinline__ int nth_near(int t, int c, int lo, int hi)
-{
-    const int below = c - lo, above = hi - c, m = min(below, above);
-    if (t <= 2 * m)
-    {
-        const int d = (t + 1) >> 1;
-        return (t & 1) ? c - d : c + d;
-    }
-    const int r = t - m;
-    return below > above ? c - r : c + r;
 }
 
 // Level l of the pyramid, read from the device-side table (a per-lane level

@@ -339,7 +339,7 @@ __device__ __forceinline__ const PGEOF_CONST Level* scalar_level(const LevelTabl
 }
 
 template <int G>
-constexpr uint32_t kGroupsOf = G <= 2 ? 8 : 12;
+constexpr uint32_t kGroupsOf = G <= 2 ? 6 : 12;
 // Streamed candidates collected in LDS before the farthest are dropped.
 constexpr uint32_t kBufGroups = 6, kBufKeys = 64 * kBufGroups;
 constexpr uint32_t kAhead = 3;  // groups of 64 of them loaded together
@@ -391,8 +391,12 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
     const uint32_t lane = threadIdx.x;
     const uint32_t k = a.k;
 
-    const uint32_t t0 = work_block(blockIdx.x, gridDim.x) * a.q_per_wave;
-    const uint32_t nq = min(a.q_per_wave, a.n_query - t0);
+    // Queries t0 .. t0 + nq.  Radius searches: the 64 / q_per_wave waves of
+    // a group look at its 64 queries first; if those are sparse, the first
+    // wave takes them all.
+    const uint32_t wave = work_block(blockIdx.x, gridDim.x), members = RADIUS ? 64u / a.q_per_wave : 1u;
+    uint32_t t0 = RADIUS ? wave / members * 64u : wave * a.q_per_wave;
+    uint32_t nq = min(RADIUS ? 64u : a.q_per_wave, a.n_query - t0);
     const uint32_t nl = uniform((uint32_t)a.tab->n_levels);
 
     // lane group l (16 lanes) looks after pyramid level l
@@ -408,18 +412,23 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
     // This lane's query.  Its region is found in float, relative to the
     // grid's origin: a cell off by one at a cell's face, or the slack of the
     // region's faces, changes no result.
-    float4 qv = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (lane < nq) qv = a.queries[t0 + lane];
-    uint64_t finite = __ballot(isfinite(qv.x) && isfinite(qv.y) && isfinite(qv.z));
-    if (RADIUS && a.limit == 0xFFFFFFFFu) finite = 0;  // no distance is below the radius
     const uint32_t limit = RADIUS ? a.limit : kNanBits;
-    const PGEOF_CONST Level* L0 = scalar_level(a.tab, 0);
-    const float relx = (float)((double)qv.x - L0->lo[0]), rely = (float)((double)qv.y - L0->lo[1]),
-                relz = (float)((double)qv.z - L0->lo[2]);
-    // rounding of a difference of such a coordinate and a cell's face
-    const float slack =
-        5e-7f * (fmaxf(fabsf(relx), fmaxf(fabsf(rely), fabsf(relz))) +
-                 (float)(L0->h * (double)max(L0->g[0], max(L0->g[1], L0->g[2]))));
+    float4 qv;
+    uint64_t finite;
+    float relx, rely, relz, slack;
+    auto load_queries = [&]() {
+        qv = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (lane < nq) qv = a.queries[t0 + lane];
+        finite = __ballot(isfinite(qv.x) && isfinite(qv.y) && isfinite(qv.z));
+        if (RADIUS && limit == 0xFFFFFFFFu) finite = 0;  // no distance is below the radius
+        const PGEOF_CONST Level* L0 = scalar_level(a.tab, 0);
+        relx = (float)((double)qv.x - L0->lo[0]), rely = (float)((double)qv.y - L0->lo[1]),
+        relz = (float)((double)qv.z - L0->lo[2]);
+        // rounding of a difference of such a coordinate and a cell's face
+        slack = 5e-7f * (fmaxf(fabsf(relx), fmaxf(fabsf(rely), fabsf(relz))) +
+                         (float)(L0->h * (double)max(L0->g[0], max(L0->g[1], L0->g[2]))));
+    };
+    load_queries();
     auto cell32 = [](float rel, float ih, int g) -> int {
         return (int)fminf(fmaxf(rel * ih, 0.0f), (float)(g - 1));
     };
@@ -448,6 +457,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
     // Sorted rows of the queries first .. first + count, `stride` keys apart
     // in LDS; lane s holds the number of keys of query first + s.
     auto write_rows = [&](uint32_t first, uint32_t count, uint32_t stride, uint32_t keys) {
+#pragma unroll 4
         for (uint32_t s = 0; s < count; ++s)
         {
             const uint32_t qorig = readlane(__float_as_uint(qv.w), first + s);
@@ -478,8 +488,8 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
 
     if constexpr (RADIUS)
     {
-        // A wave whose queries have at most 16 points around them each:
-        // one query per lane, its region's points one after the other (1 M
+        // Queries with few points around them and at most 16 hits each: one
+        // per lane, its region's points one after the other (1 M
         // uniform points with their own point in the ball: a wave per query
         // would spend its instructions on one candidate).
         const PGEOF_CONST Level* L = scalar_level(a.tab, nl - 1);
@@ -489,37 +499,62 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
         const float4* __restrict__ pts = L->pts;
         const int cx = cell32(relx, ih, a0), cy = cell32(rely, ih, a1), cz = cell32(relz, ih, a2);
         const bool mine = (finite >> lane) & 1ull;
-        uint32_t st[9], end[9], around = 0;
+        uint32_t around = 0;
 #pragma unroll
         for (int r = 0; r < 9; ++r)
         {
             const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
-            st[r] = end[r] = 0;
             if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
             {
                 const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
-                st[r] = gload(tcs, at + (uint32_t)max(cx - 1, 0));
-                end[r] = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u);
+                around += gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u) - gload(tcs, at + (uint32_t)max(cx - 1, 0));
             }
         }
-#pragma unroll
-        for (int r = 0; r < 9; ++r) around += end[r] - st[r];
         uint32_t inner, all;
         cover(cx, cy, cz, h, a0, a1, a2, inner, all);
-        if (__ballot(mine && (around > (uint32_t)kPerLane || inner < limit)) == 0)
+        // (no more than 16 around any: no more hits, the first wave's work)
+        if (wave % members && __ballot(mine && (around > (uint32_t)kPerLane || inner < limit)) == 0) return;
+        constexpr uint32_t kFew = 80;  // points a lane looks at
+        uint32_t n = 0;
+        constexpr uint32_t kSparse = (uint32_t)kPerLane + 1;
+        static_assert(64 * kSparse <= sizeof(lds) / 8, "rows of the sparse case");
+        uint64_t* row = lds + lane * kSparse;
+        if (__ballot(mine && (around > kFew || inner < limit)) == 0)
         {
-            constexpr uint32_t kSparse = (uint32_t)kPerLane + 1;
-            static_assert(64 * kSparse <= sizeof(lds) / 8, "rows of the sparse case");
-            uint64_t* row = lds + lane * kSparse;
-            uint32_t n = 0;
-#pragma unroll
+#pragma unroll 1
             for (int r = 0; r < 9; ++r)
-                for (uint32_t j = st[r]; j < end[r]; ++j)
+            {
+                const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+                uint32_t j = 0, e = 0;
+                if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
                 {
-                    const float4 p = gload(pts, j);
-                    const uint32_t d = min(__float_as_uint(sqdist32(qv.x, qv.y, qv.z, p.x, p.y, p.z)), kNanBits);
-                    if (d <= limit) row[n++] = ((uint64_t)d << 32) | __float_as_uint(p.w);
+                    const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
+                    j = gload(tcs, at + (uint32_t)max(cx - 1, 0));
+                    e = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u);
                 }
+                for (; j < e; j += 4)
+                {
+                    float4 p[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) p[u] = gload(pts, min(j + u, e - 1u));
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u)
+                    {
+                        const uint32_t d = min(__float_as_uint(sqdist32(qv.x, qv.y, qv.z, p[u].x, p[u].y, p[u].z)), kNanBits);
+                        if (j + u < e && d <= limit)
+                        {
+                            if (n < (uint32_t)kPerLane) row[n] = ((uint64_t)d << 32) | __float_as_uint(p[u].w);
+                            ++n;
+                        }
+                    }
+                }
+            }
+        }
+        else
+            n = (uint32_t)kPerLane + 1u;
+        if (__ballot(mine && n > (uint32_t)kPerLane) == 0)
+        {
+            if (wave % members) return;
             double v[kPerLane];
 #pragma unroll
             for (int r = 0; r < kPerLane; ++r) v[r] = __longlong_as_double((long long)((uint32_t)r < n ? row[r] : kNoKey));
@@ -529,6 +564,13 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
             wave_sync();
             write_rows(0, nq, kSparse, n);
             return;
+        }
+        if (members > 1)
+        {
+            t0 += wave % members * a.q_per_wave;
+            if (t0 >= a.n_query) return;
+            nq = min(a.q_per_wave, a.n_query - t0);
+            load_queries();
         }
     }
 
@@ -663,10 +705,10 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     search(std::integral_constant<int, 3>{});
                 else if (total <= 256u)
                     search(std::integral_constant<int, 4>{});
-                else if (total <= 384u)
+                else if (kGroups == 6 || total <= 384u)
                     search(std::integral_constant<int, 6>{});
-                else if (kGroups == 8 || total <= 512u)
-                    search(std::integral_constant<int, 8>{});
+                else if (total <= 512u)
+                    search(std::integral_constant<int, (kGroups > 6 ? 8 : 6)>{});
                 else
                     search(std::integral_constant<int, (int)kGroups>{});
             }
@@ -701,8 +743,10 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                 Box B{0, 0, 0, 0, 0, 0};
                 uint32_t ny = 1, nr = 1;
                 double lim = INFINITY;  // squared distance of the rows of interest
+                // rows from the query's own outwards
+                const int yc = cell_coord(qy, lo1, ih, a1), zc = cell_coord(qz, lo2, ih, a2);
                 auto row_gap2 = [&](uint32_t r, int& y, int& z) -> double {
-                    z = B.z0 + (int)(r / ny), y = B.y0 + (int)(r % ny);
+                    z = nth_near((int)(r / ny), zc, B.z0, B.z1), y = nth_near((int)(r % ny), yc, B.y0, B.y1);
                     const double dz = axis_gap(qz, z, lo2, h, margin), dy = axis_gap(qy, y, lo1, h, margin);
                     return dz * dz + dy * dy;
                 };
@@ -723,6 +767,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     B.z0 = (int)uniform((uint32_t)B.z0), B.z1 = (int)uniform((uint32_t)B.z1);
                     ny = (uint32_t)(B.y1 - B.y0 + 1), nr = ny * (uint32_t)(B.z1 - B.z0 + 1);
                     uint32_t n_buf = 0;
+                    bool again = false;
                     // the nearest of the collected keys stay (at least k, at
                     // most kMost of them), tau drops to their threshold
                     auto reduce = [&]() {
@@ -743,7 +788,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     };
                     // one row of cells per lane, then the rows' points as one
                     // list spread over the lanes, kAhead groups loaded together
-                    for (uint32_t r0 = 0; r0 < nr; r0 += 64)
+                    for (uint32_t r0 = 0; r0 < nr && !again; r0 += 64)
                     {
                         uint32_t st = 0, len = 0;
                         const uint32_t r = r0 + lane;
@@ -786,9 +831,17 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                                 if (in) buf[n_buf + lanes_below(m)] = ((uint64_t)d[u] << 32) | id[u];
                                 n_buf += (uint32_t)__popcll(m);
                             }
-                            if (n_buf > kBufKeys - 64u * kAhead) reduce();
+                            if (n_buf > kBufKeys - 64u * kAhead)
+                            {
+                                reduce();
+                                // k points lie within the new tau: with much
+                                // of the old ball left, start over with it
+                                again = 2.0f * __uint_as_float(tau) < w && (r0 + 64 < nr || tot - f0 > 1024u);
+                                if (again) break;
+                            }
                         }
                     }
+                    if (again) continue;
                     if (n_buf > kMost) reduce();
                     n = n_buf;
                     if (n >= k || tau >= limit) break;
@@ -879,7 +932,8 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
 template <int G>
 hipError_t launch_wave_g(int mode, const WaveArgs& a, hipStream_t s)
 {
-    const uint32_t nb = (a.n_query + a.q_per_wave - 1) / a.q_per_wave;
+    const bool radius = mode == kModeRadius || mode == kModeRadiusCsr;
+    const uint32_t nb = radius ? (a.n_query + 63) / 64 * (64 / a.q_per_wave) : (a.n_query + a.q_per_wave - 1) / a.q_per_wave;
     switch (mode)
     {
         case kModeKnn: k_wave_search<kModeKnn, G><<<nb, 64, 0, s>>>(a); break;
@@ -897,7 +951,8 @@ hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s)
 {
     static const char* names[4] = {"knn_search", "radius_search", "knn_features_fused", "radius_search_csr"};
     if (a.n_query == 0) return hipSuccess;
-    if (mode < 0 || mode > 3 || a.k < 1 || a.k > kWaveMaxK || a.q_per_wave < 1 || a.q_per_wave > 64)
+    if (mode < 0 || mode > 3 || a.k < 1 || a.k > kWaveMaxK || a.q_per_wave < 1 || a.q_per_wave > 64 ||
+        ((mode & 1) && 64 % a.q_per_wave))
         return hipErrorInvalidValue;
     ProfScope ps(names[mode], s);
     // rows of up to 16 G kept candidates, at least about a fifth more than k:

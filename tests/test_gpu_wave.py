@@ -177,6 +177,17 @@ def test_radius_shapes(name, r, cap):
     _radius_both(xyz, xyz, r, cap)
 
 
+# 2, 8, 32 and 64 queries per wave; sparse ones (one per lane, up to 16 hits)
+# are shared by the waves of 64 queries, the last wave being short
+@pytest.mark.parametrize("n", [4_099, 16_421, 65_601, 2_097_219])
+@pytest.mark.parametrize("hits", [2, 12, 30])
+def test_radius_waves(n, hits):
+    xyz = scenes.uniform_cube(n, seed=hits)
+    xyz[n // 2 : n // 2 + 40] = xyz[0]  # a dense spot among them
+    edge = float(np.ptp(xyz[:, 0]))
+    _radius_both(xyz, xyz, edge * float(np.cbrt(hits / (4.19 * n))), 30)
+
+
 @pytest.mark.parametrize("r", [0.0, 1e-30, np.inf, -0.5])
 def test_radius_values(r):
     xyz = scenes.uniform_cube(2000, seed=8)
