@@ -479,6 +479,13 @@ struct SearchWs
 };
 
 constexpr uint32_t kBboxBlocks = 1024;
+// Clouds up to this size sort into all levels of the pyramid from the caller's
+// order, four launches less; past it the coarse levels follow from level 0's
+// order, whose runs take one atomic each where a LiDAR scan's hot cells take
+// one per point (us per kNN call, k = 20, at once / from level 0: 30 k points
+// 84 / 85 uniform, 181 / 180 LiDAR; 60 k 112 / 127, 236 / 241; 100 k 125 / 137,
+// 315 / 298; 200 k 193 / 195, 372 / 347; another 100 k LiDAR cloud 385 / 287).
+constexpr uint32_t kSmallBuild = 1u << 16;
 
 struct HeapPlan
 {
@@ -550,7 +557,7 @@ size_t search_ws_bytes(uint64_t n, uint64_t m, uint32_t k, bool csr)
     const uint64_t G = grid_cap(n) + 1;
     size_t b = 0;
     b += al(kBboxBlocks * 6 * sizeof(float)) + al(64) + al(64);
-    b += al(G * 4) + al((2 * G + 64) * 4) + al(scan_partials_needed(G + 64) * 4);
+    b += al((G + 4) * 4) + al((2 * G + 64) * 4) + al((scan_partials_needed(2 * G + 64) + 8) * 4);
     b += 2 * al(n * 4) + kMaxLevels * al(n * 16);
     b += 2 * al(m * 4) + al(m * 16);
     b += 2 * al((m + 1) * 4) + al(scan_partials_needed(m + 1) * 4) + 2 * al(m * 16) + 3 * al(m * 4);
@@ -568,9 +575,9 @@ SearchWs carve(Arena& ar, uint64_t n, uint64_t m, uint32_t k, bool csr)
     w.bbox_partial = ar.take<float>(kBboxBlocks * 6);
     w.bbox_out = ar.take<float>(16);
     w.sumsq = ar.take<unsigned long long>(8);
-    w.count = ar.take<uint32_t>(G);
+    w.count = ar.take<uint32_t>(G + 4);
     w.cs_all = ar.take<uint32_t>(2 * G + 64);
-    w.scan_part = ar.take<uint32_t>(scan_partials_needed(G + 64));
+    w.scan_part = ar.take<uint32_t>(scan_partials_needed(2 * G + 64) + 8);
     w.cell = ar.take<uint32_t>(n);
     w.rank = ar.take<uint32_t>(n);
     for (int l = 0; l < kMaxLevels; ++l) w.pts[l] = ar.take<float4>(n);
@@ -676,40 +683,72 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
     p.knn_cell_points_max = t.knn_cell_points_max;
     p.radius_cell_factor = t.radius_cell_factor;
     p.level_ratio = t.grid_level_ratio;
-    p.probe_stride = std::max<uint32_t>(1, std::min<uint32_t>(64, n >> 20));
+    // the sizing probe counts some 32,768 of the points: 1 M of them took
+    // 58 us of hot-cell atomics where this takes 12
+    p.probe_stride = std::max<uint32_t>(1, n >> 15);
     level_tables(w.cs_all, cap, p.cs, p.cs_room);
     for (int l = 0; l < kMaxLevels; ++l) p.pts[l] = w.pts[l];
 
     const uint32_t nbb = std::max<uint32_t>(1, std::min<uint32_t>(kBboxBlocks, (n + 255) / 256));
-    HIP_TRY(launch_bbox(data, n, w.bbox_partial, nbb, w.tab->bb, s));
-    HIP_TRY(launch_plan_probe(p, w.tab, s));
+    HIP_TRY(launch_bbox_plan(data, p, w.bbox_partial, nbb, w.tab, s));
     if (!is_radius) HIP_TRY(launch_probe(data, n, p.probe_stride, w.tab, w.count, cap + 1, s));
     HIP_TRY(launch_plan_levels(p, w.tab, s));
-    for (int l = 0; l < p.max_levels; ++l)
+
+    // Counting sort into the levels.  Counts go straight into the level's
+    // table, scanned in place.  With the last level's points unused they hold
+    // the coarser levels' cells and ranks, and several levels share each
+    // launch: all of them from the caller's points for small clouds, where
+    // launches count, else level 0 first and the coarser ones from its order
+    // (runs of equal cells, one atomic each).
+    const int L = p.max_levels;
+    LevelSet v{};
+    uint64_t part = 0;
+    for (int l = 0; l < kMaxLevels; ++l)
     {
-        // counts straight into the level's table, scanned in place
-        uint32_t* csl = p.cs[l];
-        const uint64_t* G = &w.tab->G[l];
-        HIP_TRY(launch_fill_u32_dyn(csl, p.cs_room[l], G, 1, 0u, s));
-        if (l == 0)
-            HIP_TRY(launch_hist(data, n, w.tab, 0, csl, w.cell, w.rank, s));
-        else  // from the level-0 order: runs of equal cells, one atomic each
-            HIP_TRY(launch_hist_sorted(w.pts[0], n, w.tab, l, csl, w.cell, w.rank, s));
-        HIP_TRY(launch_scan_exclusive_dyn(csl, csl, p.cs_room[l], G, 1, w.scan_part, s));
-        if (l == 0)
-            HIP_TRY(launch_scatter(data, n, w.cell, w.rank, csl, w.pts[0], w.tab, 0, s));
-        else
-            HIP_TRY(launch_scatter_sorted(w.pts[0], n, w.cell, w.rank, csl, w.pts[l], w.tab, l, s));
+        v.cs[l] = p.cs[l];
+        v.room[l] = p.cs_room[l];
+        v.pts[l] = w.pts[l];
+        const bool own = l > 0 && L < kMaxLevels;
+        uint32_t* spare = reinterpret_cast<uint32_t*>(w.pts[kMaxLevels - 1]);
+        v.cell[l] = own && l < L ? spare + (size_t)(l - 1) * 2 * n : w.cell;
+        v.rank[l] = own && l < L ? spare + (size_t)(l - 1) * 2 * n + n : w.rank;
+        v.part[l] = w.scan_part + part;
+        part += scan_partials_needed(p.cs_room[l]);
+    }
+    HIP_TRY(launch_fill_levels(v, w.tab, 0, L, s));
+    const int first = L < kMaxLevels && n <= kSmallBuild ? L : 1;
+    HIP_TRY(launch_hist(data, n, w.tab, v, 0, first, s));
+    HIP_TRY(launch_scan_levels(v, w.tab, 0, first, s));
+    HIP_TRY(launch_scatter(data, n, w.tab, v, 0, first, s));
+    for (int l = first; l < L;)
+    {
+        const int count = L < kMaxLevels ? L - l : 1;
+        HIP_TRY(launch_hist_sorted(w.pts[0], n, w.tab, v, l, count, s));
+        HIP_TRY(launch_scan_levels(v, w.tab, l, count, s));
+        HIP_TRY(launch_scatter_sorted(w.pts[0], n, w.tab, v, l, count, s));
+        l += count;
     }
     if (query == data && m == n)
         *qs_out = w.pts[0];
+    else if (wave && m <= 8192)
+    {
+        // too few queries to share cells or cache lines: in the caller's order
+        HIP_TRY(launch_pack_queries(query, m, w.qs, s));
+        *qs_out = w.qs;
+    }
     else
     {
-        const uint64_t* G0 = &w.tab->G[0];
-        HIP_TRY(launch_fill_u32_dyn(w.count, cap + 1, G0, 1, 0u, s));
-        HIP_TRY(launch_hist(query, m, w.tab, 0, w.count, w.qcell, w.qrank, s));
-        HIP_TRY(launch_scan_exclusive_dyn(w.count, w.count, cap + 1, G0, 1, w.scan_part, s));
-        HIP_TRY(launch_scatter(query, m, w.qcell, w.qrank, w.count, w.qs, w.tab, 0, s));
+        LevelSet q{};
+        q.cs[0] = w.count;
+        q.room[0] = cap + 1;
+        q.pts[0] = w.qs;
+        q.cell[0] = w.qcell;
+        q.rank[0] = w.qrank;
+        q.part[0] = w.scan_part;
+        HIP_TRY(launch_fill_levels(q, w.tab, 0, 1, s));
+        HIP_TRY(launch_hist(query, m, w.tab, q, 0, 1, s));
+        HIP_TRY(launch_scan_levels(q, w.tab, 0, 1, s));
+        HIP_TRY(launch_scatter(query, m, w.tab, q, 0, 1, s));
         *qs_out = w.qs;
     }
     sa.tab = w.tab;
@@ -720,7 +759,8 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
 // Device search core shared by the host and device entry points.
 int run_search(int mode, const float* data, uint32_t n, const float* query, uint32_t m, uint32_t k, float radius,
                void* out_idx, float* out_d2, float* out_feat, uint32_t* out_count, Arena& ar, hipStream_t s,
-               SearchWs* ws_out = nullptr, const uint32_t* scales = nullptr, uint32_t n_scales = 0)
+               SearchWs* ws_out = nullptr, const uint32_t* scales = nullptr, uint32_t n_scales = 0,
+               uint32_t* out_ptr = nullptr)
 {
     const bool csr = mode == kModeRadiusCsr || mode == kModeRadiusMulti;
     SearchWs w = carve(ar, n, m, k, csr);
@@ -789,6 +829,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         b.out_idx = (uint32_t*)a.out_idx;
         b.out_d2 = out_d2;
         b.out_feat = out_feat;
+        b.out_ptr = out_ptr;
         HIP_TRY(launch_wave_search(mode, b, s));
     }
     else if (mode == kModeKnn || mode == kModeKnnFeat)
@@ -847,6 +888,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     }
     else
         HIP_TRY(launch_search(mode, a, hp.block, hp.lds, hp.global, false, s));
+    if (out_ptr && !wave) HIP_TRY(launch_arange_ptr(out_ptr, m, k, s));
     if (ws_out) *ws_out = w;
     return PGEOF_OK;
 }
@@ -1381,11 +1423,8 @@ int pgeof_knn_features_device(const float* xyz, int64_t n, uint32_t knn, uint32_
     Arena ar;
     rc = acquire_ws(g, workspace, workspace_bytes, pgeof_knn_workspace_size(n, n, knn), s, ar);
     if (rc) return rc;
-    rc = run_search(kModeKnnFeat, xyz, (uint32_t)n, xyz, (uint32_t)n, knn, 0.0f, nn, sqr_dist, features, nullptr, ar,
-                    s);
-    if (rc) return rc;
-    HIP_TRY(launch_arange_ptr(nn_ptr, (uint32_t)n, knn, s));
-    return PGEOF_OK;
+    return run_search(kModeKnnFeat, xyz, (uint32_t)n, xyz, (uint32_t)n, knn, 0.0f, nn, sqr_dist, features, nullptr, ar,
+                      s, nullptr, nullptr, 0, nn_ptr);
 }
 
 int pgeof_radius_csr_device(const float* xyz, int64_t n, float search_radius, uint32_t max_knn, uint32_t* nn,

@@ -136,6 +136,7 @@ struct WaveArgs
     uint32_t* out_idx;      // (n_query, k), rows = original query index
     float* out_d2;          // (n_query, k) or nullptr
     float* out_feat;        // (n_query, 11), fused features
+    uint32_t* out_ptr;      // (n_query + 1), fused features: row offsets of the CSR
     uint32_t* out_count;    // radius: hits per original query (at most k) or nullptr
 };
 constexpr uint32_t kWaveMaxK = 108;  // largest k of that kernel (128 kept candidates per query)
@@ -174,24 +175,40 @@ hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, 
                                  hipStream_t s);
 hipError_t launch_scan_exclusive_dyn(const uint32_t* in, uint32_t* out, uint64_t n_max, const uint64_t* n_dev,
                                      uint64_t add, uint32_t* partials, hipStream_t s);
-// Grid planning on the device: pgeof_plan_probe after the bounding box (into
-// tab->bb), pgeof_plan_levels after the probe histogram's sum of squares.
-hipError_t launch_plan_probe(const PlanArgs& p, LevelTable* tab, hipStream_t s);
+// Grid planning on the device: launch_bbox_plan finds the bounding box (into
+// tab->bb) and plans the probe, launch_plan_levels follows the probe
+// histogram's sum of squares.
+hipError_t launch_bbox_plan(const float* xyz, const PlanArgs& p, float* partial, uint32_t n_partial, LevelTable* tab,
+                            hipStream_t s);
 hipError_t launch_plan_levels(const PlanArgs& p, LevelTable* tab, hipStream_t s);
 // cell counts of every stride-th point at the probe grid, and their sum of squares
 hipError_t launch_probe(const float* xyz, uint32_t n, uint32_t stride, LevelTable* tab, uint32_t* count,
                         uint64_t count_room, hipStream_t s);
-// counting sort of points into level l (level 0 from xyz, l > 0 from the
-// level-0 array, already sorted by a finer grid); nothing when the level is absent
-hipError_t launch_hist(const float* xyz, uint32_t n, const LevelTable* tab, int l, uint32_t* count, uint32_t* cell,
-                       uint32_t* rank, hipStream_t s);
-hipError_t launch_hist_sorted(const float4* pts, uint32_t n, const LevelTable* tab, int l, uint32_t* count,
-                              uint32_t* cell, uint32_t* rank, hipStream_t s);
-hipError_t launch_scatter(const float* xyz, uint32_t n, const uint32_t* cell, const uint32_t* rank,
-                          const uint32_t* cell_start, float4* pts, const LevelTable* tab, int l, hipStream_t s);
-hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const uint32_t* cell, const uint32_t* rank,
-                                 const uint32_t* cell_start, float4* out, const LevelTable* tab, int l,
-                                 hipStream_t s);
+
+// Tables of a counting sort into several levels of the grid at once (levels
+// l0 .. l0 + n_levels of a launch; absent levels of the table do nothing).
+struct LevelSet
+{
+    uint32_t* cs[kMaxLevels];    // cell counts, scanned in place into cell starts
+    uint64_t room[kMaxLevels];   // entries available there
+    float4* pts[kMaxLevels];     // the sorted points
+    uint32_t* cell[kMaxLevels];  // per point: cell, and rank in it
+    uint32_t* rank[kMaxLevels];
+    uint32_t* part[kMaxLevels];  // scan partials
+};
+hipError_t launch_fill_levels(const LevelSet& v, const LevelTable* tab, int l0, int n_levels, hipStream_t s);
+// from the caller's points, or (sorted) from the level-0 array
+hipError_t launch_hist(const float* xyz, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0, int n_levels,
+                       hipStream_t s);
+hipError_t launch_hist_sorted(const float4* pts, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0,
+                              int n_levels, hipStream_t s);
+hipError_t launch_scan_levels(const LevelSet& v, const LevelTable* tab, int l0, int n_levels, hipStream_t s);
+hipError_t launch_scatter(const float* xyz, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0, int n_levels,
+                          hipStream_t s);
+hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0,
+                                 int n_levels, hipStream_t s);
+// queries as (x, y, z, index), in the caller's order
+hipError_t launch_pack_queries(const float* q, uint32_t m, float4* out, hipStream_t s);
 hipError_t launch_search(int mode, const SearchArgs& a, int block, size_t lds_bytes, bool global_heap, bool budget,
                          hipStream_t s);
 hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s);  // pgeof_wave.hip

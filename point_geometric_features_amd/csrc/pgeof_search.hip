@@ -67,8 +67,8 @@ __global__ __launch_bounds__(256) void k_bbox(const float* __restrict__ xyz, uin
     if (threadIdx.x < 6) partial[blockIdx.x * 6 + threadIdx.x] = s[threadIdx.x][0];
 }
 
-__global__ __launch_bounds__(256) void k_bbox_final(const float* __restrict__ partial, uint32_t np,
-                                                    float* __restrict__ out6)
+// one block of 256 threads: the bounding box of all blocks' partial ones
+__device__ __forceinline__ void bbox_reduce(const float* __restrict__ partial, uint32_t np, float* __restrict__ out6)
 {
     float mn[3] = {INFINITY, INFINITY, INFINITY}, mx[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (uint32_t b = threadIdx.x; b < np; b += 256)
@@ -95,6 +95,12 @@ __global__ __launch_bounds__(256) void k_bbox_final(const float* __restrict__ pa
         __syncthreads();
     }
     if (threadIdx.x < 6) out6[threadIdx.x] = s[threadIdx.x][0];
+}
+
+__global__ __launch_bounds__(256) void k_bbox_final(const float* __restrict__ partial, uint32_t np,
+                                                    float* __restrict__ out6)
+{
+    bbox_reduce(partial, np, out6);
 }
 
 // ---------------------------------------------------------- fill / ptr ----
@@ -139,16 +145,32 @@ __device__ __forceinline__ uint32_t cell_id(const Level& L, double x, double y, 
     return ((uint32_t)cz * (uint32_t)L.g[1] + (uint32_t)cy) * (uint32_t)L.g[0] + (uint32_t)cx;
 }
 
-// Counting-sort histogram, 16 points per thread; rank = the point's rank in
+// Cell counts of the levels from l0 (one per block row) to zero, the total's
+// slot included.
+__global__ __launch_bounds__(256) void k_fill_levels(LevelSet v, const LevelTable* __restrict__ tab, int l0)
+{
+    const int l = l0 + (int)blockIdx.y;
+    const uint64_t G = tab->G[l];
+    if (G == 0) return;
+    uint4* __restrict__ p4 = reinterpret_cast<uint4*>(v.cs[l]);  // tables are 16-byte aligned, their rooms whole uint4
+    const uint64_t n4 = (min(G + 1, v.room[l]) + 3) / 4;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n4; i += (uint64_t)gridDim.x * 256)
+        p4[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// Counting-sort histogram, kPer points per thread; rank = the point's rank in
 // its cell.  Grids of few cells count per block in LDS first (one global
 // atomic per touched cell and block: a few hot cells would otherwise
 // serialise the atomics), larger ones count in global memory directly.
 constexpr uint32_t kSmallHistCells = 8192;
+template <uint32_t kPer>
 __global__ __launch_bounds__(256) void k_hist(const float* __restrict__ xyz, uint32_t n,
-                                              const LevelTable* __restrict__ tab, int l,
-                                              uint32_t* __restrict__ count, uint32_t* __restrict__ cell,
-                                              uint32_t* __restrict__ rank)
+                                              const LevelTable* __restrict__ tab, LevelSet v, int l0)
 {
+    const int l = l0 + (int)blockIdx.y;
+    uint32_t* __restrict__ count = v.cs[l];
+    uint32_t* __restrict__ cell = v.cell[l];
+    uint32_t* __restrict__ rank = v.rank[l];
     __shared__ uint32_t bins[kSmallHistCells];
     const uint64_t G = cells_of(tab, l);
     if (G == 0) return;
@@ -159,7 +181,6 @@ __global__ __launch_bounds__(256) void k_hist(const float* __restrict__ xyz, uin
         for (uint32_t c = threadIdx.x; c < (uint32_t)G; c += 256) bins[c] = 0;
         __syncthreads();
     }
-    constexpr uint32_t kPer = 16;  // points per thread
     const uint64_t base = (uint64_t)blockIdx.x * 256 * kPer;
     uint32_t cid[kPer], lr[kPer];
 #pragma unroll
@@ -203,10 +224,12 @@ __global__ __launch_bounds__(256) void k_hist(const float* __restrict__ xyz, uin
 // within a wave takes one atomic for the whole run.  rank = the run's base +
 // the lane's offset in the run; cell/rank are indexed by sorted position.
 __global__ __launch_bounds__(256) void k_hist_sorted(const float4* __restrict__ pts, uint32_t n,
-                                                     const LevelTable* __restrict__ tab, int l,
-                                                     uint32_t* __restrict__ count, uint32_t* __restrict__ cell,
-                                                     uint32_t* __restrict__ rank)
+                                                     const LevelTable* __restrict__ tab, LevelSet v, int l0)
 {
+    const int l = l0 + (int)blockIdx.y;
+    uint32_t* __restrict__ count = v.cs[l];
+    uint32_t* __restrict__ cell = v.cell[l];
+    uint32_t* __restrict__ rank = v.rank[l];
     if (cells_of(tab, l) == 0) return;
     const Level L = level_of(tab, l);
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
@@ -239,15 +262,12 @@ __global__ __launch_bounds__(256) void k_hist_sorted(const float4* __restrict__ 
 }
 
 __global__ __launch_bounds__(256) void k_scatter_sorted(const float4* __restrict__ in, uint32_t n,
-                                                        const uint32_t* __restrict__ cell,
-                                                        const uint32_t* __restrict__ rank,
-                                                        const uint32_t* __restrict__ cell_start,
-                                                        float4* __restrict__ out, const LevelTable* __restrict__ tab,
-                                                        int l)
+                                                        const LevelTable* __restrict__ tab, LevelSet v, int l0)
 {
+    const int l = l0 + (int)blockIdx.y;
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n || cells_of(tab, l) == 0) return;
-    out[cell_start[cell[i]] + rank[i]] = in[i];
+    v.pts[l][v.cs[l][v.cell[l][i]] + v.rank[l][i]] = in[i];
 }
 
 // Cell counts of every `stride`-th point at the probe grid (grid sizing estimate only).
@@ -343,8 +363,11 @@ __device__ void plan_extent(const float bb[6], double ext[3], double& emax)
 
 // After the bounding box: the grid-size floor, and for kNN the probe grid of
 // the first guess of h (points per cell T, assuming a uniformly filled box).
-__global__ void k_plan_probe(PlanArgs p, LevelTable* __restrict__ tab)
+__global__ __launch_bounds__(256) void k_bbox_plan(const float* __restrict__ partial, uint32_t np, PlanArgs p,
+                                                   LevelTable* __restrict__ tab)
 {
+    bbox_reduce(partial, np, tab->bb);
+    __syncthreads();
     if (threadIdx.x != 0) return;
     float bb[6];
     bool finite = true;
@@ -401,7 +424,7 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         h = isfinite(r) && r > 0.0 ? r * p.radius_cell_factor : emax;
         if (p.wave && isfinite(r) && r > 0.0)
         {
-            // the coarsest level's cells span the radius (a little more, for
+            // the coarser level's cells span the radius (a little more, for
             // the float region tests), so that 3x3x3 of them hold the ball;
             // one of half their edge, or as fine as the cap allows, serves
             // the dense parts
@@ -488,15 +511,12 @@ __device__ __forceinline__ uint4 scan_load4(const uint32_t* in, uint64_t i, uint
     return v;
 }
 
-// The three scan kernels loop over the tiles (a block takes tiles b, b +
-// grid, ...), so that a launch sized for the largest input does no empty
-// work when the device-side count is smaller.
+// The scan kernels loop over the tiles (a block takes tiles b, b + grid,
+// ...), so that a launch sized for the largest input does no empty work when
+// the device-side count is smaller.
 template <bool VEC>
-__global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n_max,
-                                                            const uint64_t* __restrict__ n_dev, uint64_t add,
-                                                            uint32_t* __restrict__ partials)
+__device__ __forceinline__ void scan_reduce(const uint32_t* __restrict__ in, uint64_t n, uint32_t* __restrict__ partials)
 {
-    const uint64_t n = dyn_count(n_max, n_dev, add);
     const uint64_t nt = (n + kScanTile - 1) / kScanTile;
     for (uint64_t tile = blockIdx.x; tile < nt; tile += gridDim.x)
     {
@@ -513,10 +533,9 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const uint32_t* __re
     }
 }
 
-__global__ __launch_bounds__(kScanBlock) void k_scan_partials(uint32_t* __restrict__ partials, uint64_t n_max,
-                                                              const uint64_t* __restrict__ n_dev, uint64_t add)
+__device__ __forceinline__ void scan_partials(uint32_t* __restrict__ partials, uint64_t n)
 {
-    const uint32_t nt = (uint32_t)((dyn_count(n_max, n_dev, add) + kScanTile - 1) / kScanTile);
+    const uint32_t nt = (uint32_t)((n + kScanTile - 1) / kScanTile);
     uint32_t carry = 0;
     for (uint32_t base = 0; base < nt; base += kScanTile)
     {
@@ -540,17 +559,25 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_partials(uint32_t* __restri
     }
 }
 
-template <bool VEC>
-__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const uint32_t* in, uint32_t* out, uint64_t n_max,
-                                                           const uint64_t* __restrict__ n_dev, uint64_t add,
-                                                           const uint32_t* __restrict__ partials)
+// SUMS: the partials are the tiles' sums, not yet scanned: a block adds up
+// the ones before its tile itself
+template <bool VEC, bool SUMS>
+__device__ __forceinline__ void scan_apply(const uint32_t* in, uint32_t* out, uint64_t n,
+                                           const uint32_t* __restrict__ partials)
 {
-    const uint64_t n = dyn_count(n_max, n_dev, add);
     const uint64_t nt = (n + kScanTile - 1) / kScanTile;
     for (uint64_t tile = blockIdx.x; tile < nt; tile += gridDim.x)
     {
         const uint64_t base = tile * kScanTile;
-        uint32_t carry = partials[tile];
+        uint32_t carry = 0;
+        if (SUMS)
+        {
+            uint32_t mine = 0;
+            for (uint64_t t = threadIdx.x; t < tile; t += kScanBlock) mine += partials[t];
+            block_exclusive_scan(mine, carry);
+        }
+        else
+            carry = partials[tile];
         for (int sub = 0; sub < kScanTile; sub += 4 * kScanBlock)
         {
             const uint64_t i = base + sub + 4 * threadIdx.x;
@@ -572,16 +599,64 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const uint32_t* in, u
     }
 }
 
+template <bool VEC>
+__global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const uint32_t* __restrict__ in, uint64_t n_max,
+                                                            const uint64_t* __restrict__ n_dev, uint64_t add,
+                                                            uint32_t* __restrict__ partials)
+{
+    scan_reduce<VEC>(in, dyn_count(n_max, n_dev, add), partials);
+}
+__global__ __launch_bounds__(kScanBlock) void k_scan_partials(uint32_t* __restrict__ partials, uint64_t n_max,
+                                                              const uint64_t* __restrict__ n_dev, uint64_t add)
+{
+    scan_partials(partials, dyn_count(n_max, n_dev, add));
+}
+template <bool VEC, bool SUMS>
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const uint32_t* in, uint32_t* out, uint64_t n_max,
+                                                           const uint64_t* __restrict__ n_dev, uint64_t add,
+                                                           const uint32_t* __restrict__ partials)
+{
+    scan_apply<VEC, SUMS>(in, out, dyn_count(n_max, n_dev, add), partials);
+}
+
+// the same over the cell counts of several levels (one per block row)
+__device__ __forceinline__ uint64_t level_entries(const LevelTable* tab, const LevelSet& v, int l)
+{
+    const uint64_t G = tab->G[l];
+    return G ? min(G + 1, v.room[l]) : 0;
+}
+__global__ __launch_bounds__(kScanBlock) void k_scan_levels_reduce(LevelSet v, const LevelTable* __restrict__ tab, int l0)
+{
+    const int l = l0 + (int)blockIdx.y;
+    scan_reduce<true>(v.cs[l], level_entries(tab, v, l), v.part[l]);
+}
+__global__ __launch_bounds__(kScanBlock) void k_scan_levels_partials(LevelSet v, const LevelTable* __restrict__ tab, int l0)
+{
+    const int l = l0 + (int)blockIdx.y;
+    scan_partials(v.part[l], level_entries(tab, v, l));
+}
+template <bool SUMS>
+__global__ __launch_bounds__(kScanBlock) void k_scan_levels_apply(LevelSet v, const LevelTable* __restrict__ tab, int l0)
+{
+    const int l = l0 + (int)blockIdx.y;
+    scan_apply<true, SUMS>(v.cs[l], v.cs[l], level_entries(tab, v, l), v.part[l]);
+}
+
 // ------------------------------------------------------------ scatter ----
 __global__ __launch_bounds__(256) void k_scatter(const float* __restrict__ xyz, uint32_t n,
-                                                 const uint32_t* __restrict__ cell, const uint32_t* __restrict__ rank,
-                                                 const uint32_t* __restrict__ cell_start, float4* __restrict__ pts,
-                                                 const LevelTable* __restrict__ tab, int l)
+                                                 const LevelTable* __restrict__ tab, LevelSet v, int l0)
 {
+    const int l = l0 + (int)blockIdx.y;
     const uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n || cells_of(tab, l) == 0) return;
-    const uint32_t pos = cell_start[cell[i]] + rank[i];
-    pts[pos] = make_float4(xyz[i * 3 + 0], xyz[i * 3 + 1], xyz[i * 3 + 2], __uint_as_float((uint32_t)i));
+    const uint32_t pos = v.cs[l][v.cell[l][i]] + v.rank[l][i];
+    v.pts[l][pos] = make_float4(xyz[i * 3 + 0], xyz[i * 3 + 1], xyz[i * 3 + 2], __uint_as_float((uint32_t)i));
+}
+
+__global__ __launch_bounds__(256) void k_pack_queries(const float* __restrict__ q, uint32_t m, float4* __restrict__ out)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < m) out[i] = make_float4(q[i * 3 + 0], q[i * 3 + 1], q[i * 3 + 2], __uint_as_float(i));
 }
 
 __global__ __launch_bounds__(256) void k_compact_rows(const uint32_t* __restrict__ dense, uint32_t n_rows,
@@ -2325,9 +2400,12 @@ hipError_t launch_put_u32(uint32_t* p, const uint64_t* n_dev, uint32_t v, hipStr
     return hipGetLastError();
 }
 
-hipError_t launch_plan_probe(const PlanArgs& p, LevelTable* tab, hipStream_t s)
+hipError_t launch_bbox_plan(const float* xyz, const PlanArgs& p, float* partial, uint32_t n_partial, LevelTable* tab,
+                            hipStream_t s)
 {
-    k_plan_probe<<<1, 64, 0, s>>>(p, tab);
+    ProfScope ps("bbox", s);
+    k_bbox<<<n_partial, 256, 0, s>>>(xyz, p.n, partial);
+    k_bbox_plan<<<1, 256, 0, s>>>(partial, n_partial, p, tab);
     return hipGetLastError();
 }
 
@@ -2343,12 +2421,17 @@ hipError_t launch_arange_ptr(uint32_t* nn_ptr, uint32_t n_points, uint32_t k, hi
     return hipGetLastError();
 }
 
-hipError_t launch_hist(const float* xyz, uint32_t n, const LevelTable* tab, int l, uint32_t* count, uint32_t* cell,
-                       uint32_t* rank, hipStream_t s)
+hipError_t launch_hist(const float* xyz, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0, int n_levels,
+                       hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     ProfScope ps("grid_histogram", s);
-    k_hist<<<(n + 256 * 16 - 1) / (256 * 16), 256, 0, s>>>(xyz, n, tab, l, count, cell, rank);
+    // 16 points per thread share the LDS bins of a large cloud; up to 2^18 they
+    // would leave the chip short of blocks (10 k points: 8.5 us, with 4 5.6)
+    if (n <= (1u << 18))
+        k_hist<4><<<dim3((n + 256 * 4 - 1) / (256 * 4), (uint32_t)n_levels), 256, 0, s>>>(xyz, n, tab, v, l0);
+    else
+        k_hist<16><<<dim3((n + 256 * 16 - 1) / (256 * 16), (uint32_t)n_levels), 256, 0, s>>>(xyz, n, tab, v, l0);
     return hipGetLastError();
 }
 
@@ -2448,6 +2531,11 @@ hipError_t launch_compact_queries(const float4* q, uint32_t n_max, const uint64_
     return hipGetLastError();
 }
 
+// Up to kSumTiles tiles the apply kernel adds up the tiles' sums itself: one
+// launch less (about 3 us of a small call); a launch sized for more (the
+// tables of over 1 M points) would read megabytes of partials.
+constexpr uint64_t kSumTiles = 2048;
+
 size_t scan_partials_needed(uint64_t n) { return (size_t)((n + kScanTile - 1) / kScanTile) + 1; }
 
 hipError_t launch_scan_exclusive(const uint32_t* in, uint32_t* out, uint64_t n, uint32_t* partials, hipStream_t s)
@@ -2467,11 +2555,19 @@ hipError_t launch_scan_exclusive_dyn(const uint32_t* in, uint32_t* out, uint64_t
         k_scan_reduce<true><<<nb, kScanBlock, 0, s>>>(in, n_max, n_dev, add, partials);
     else
         k_scan_reduce<false><<<nb, kScanBlock, 0, s>>>(in, n_max, n_dev, add, partials);
+    if (nt <= kSumTiles)
+    {
+        if (vec)
+            k_scan_apply<true, true><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
+        else
+            k_scan_apply<false, true><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
+        return hipGetLastError();
+    }
     k_scan_partials<<<1, kScanBlock, 0, s>>>(partials, n_max, n_dev, add);
     if (vec)
-        k_scan_apply<true><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
+        k_scan_apply<true, false><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
     else
-        k_scan_apply<false><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
+        k_scan_apply<false, false><<<nb, kScanBlock, 0, s>>>(in, out, n_max, n_dev, add, partials);
     return hipGetLastError();
 }
 
@@ -2484,35 +2580,64 @@ hipError_t launch_probe(const float* xyz, uint32_t n, uint32_t stride, LevelTabl
     hipError_t e = launch_fill_u32_dyn(count, count_room, &tab->probe_G, 0, 0u, s);
     if (e != hipSuccess) return e;
     k_hist_probe<<<(ns + 255) / 256, 256, 0, s>>>(xyz, n, stride, tab, count);
-    k_sumsq<<<blocks_for(count_room, 256, 2048), 256, 0, s>>>(count, tab);
+    // (each block ends in one atomic on the same word: 2048 of them took 26 us)
+    k_sumsq<<<blocks_for(count_room, 256, 128), 256, 0, s>>>(count, tab);
     return hipGetLastError();
 }
 
-hipError_t launch_hist_sorted(const float4* pts, uint32_t n, const LevelTable* tab, int l, uint32_t* count,
-                              uint32_t* cell, uint32_t* rank, hipStream_t s)
+hipError_t launch_hist_sorted(const float4* pts, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0,
+                              int n_levels, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     ProfScope ps("grid_histogram_sorted", s);
-    k_hist_sorted<<<(n + 255) / 256, 256, 0, s>>>(pts, n, tab, l, count, cell, rank);
+    k_hist_sorted<<<dim3((n + 255) / 256, (uint32_t)n_levels), 256, 0, s>>>(pts, n, tab, v, l0);
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const uint32_t* cell, const uint32_t* rank,
-                                 const uint32_t* cell_start, float4* out, const LevelTable* tab, int l,
-                                 hipStream_t s)
+hipError_t launch_scatter_sorted(const float4* in, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0,
+                                 int n_levels, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     ProfScope ps("grid_scatter", s);
-    k_scatter_sorted<<<(n + 255) / 256, 256, 0, s>>>(in, n, cell, rank, cell_start, out, tab, l);
+    k_scatter_sorted<<<dim3((n + 255) / 256, (uint32_t)n_levels), 256, 0, s>>>(in, n, tab, v, l0);
     return hipGetLastError();
 }
 
-hipError_t launch_scatter(const float* xyz, uint32_t n, const uint32_t* cell, const uint32_t* rank,
-                          const uint32_t* cell_start, float4* pts, const LevelTable* tab, int l, hipStream_t s)
+hipError_t launch_scatter(const float* xyz, uint32_t n, const LevelTable* tab, const LevelSet& v, int l0, int n_levels,
+                          hipStream_t s)
 {
     if (n == 0) return hipSuccess;
     ProfScope ps("grid_scatter", s);
-    k_scatter<<<(n + 255) / 256, 256, 0, s>>>(xyz, n, cell, rank, cell_start, pts, tab, l);
+    k_scatter<<<dim3((n + 255) / 256, (uint32_t)n_levels), 256, 0, s>>>(xyz, n, tab, v, l0);
+    return hipGetLastError();
+}
+
+hipError_t launch_fill_levels(const LevelSet& v, const LevelTable* tab, int l0, int n_levels, hipStream_t s)
+{
+    k_fill_levels<<<dim3(blocks_for(v.room[l0], 1024, 4096), (uint32_t)n_levels), 256, 0, s>>>(v, tab, l0);
+    return hipGetLastError();
+}
+
+hipError_t launch_scan_levels(const LevelSet& v, const LevelTable* tab, int l0, int n_levels, hipStream_t s)
+{
+    ProfScope ps("grid_scan", s);
+    const uint64_t nt = (v.room[l0] + kScanTile - 1) / kScanTile;
+    const dim3 grid((uint32_t)std::min<uint64_t>(nt, 2048), (uint32_t)n_levels);
+    k_scan_levels_reduce<<<grid, kScanBlock, 0, s>>>(v, tab, l0);
+    if (nt <= kSumTiles)
+        k_scan_levels_apply<true><<<grid, kScanBlock, 0, s>>>(v, tab, l0);
+    else
+    {
+        k_scan_levels_partials<<<dim3(1, (uint32_t)n_levels), kScanBlock, 0, s>>>(v, tab, l0);
+        k_scan_levels_apply<false><<<grid, kScanBlock, 0, s>>>(v, tab, l0);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_queries(const float* q, uint32_t m, float4* out, hipStream_t s)
+{
+    if (m == 0) return hipSuccess;
+    k_pack_queries<<<(m + 255) / 256, 256, 0, s>>>(q, m, out);
     return hipGetLastError();
 }
 

@@ -887,6 +887,9 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
         // accumulated ----
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
         if (lane >= nq) return;
+        // this wave's share of the CSR row offsets
+        a.out_ptr[t0 + lane] = (t0 + lane) * k;
+        if (t0 + lane == a.n_query - 1) a.out_ptr[a.n_query] = a.n_query * k;
         float f[11];
         if ((finite >> lane) & 1ull)
         {

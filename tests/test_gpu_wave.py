@@ -231,6 +231,34 @@ def test_radius_csr(r):
     np.testing.assert_array_equal(out[0][2], out[1][2])
 
 
+# the grid's levels are built at once or after level 0 (65,536 points), with 4
+# or 16 points per thread (262,144), and few queries stay unsorted (8,192)
+@pytest.mark.parametrize("n", [65_535, 65_536, 65_537, 262_144, 262_145])
+@pytest.mark.parametrize("m", [8_192, 8_193])
+@pytest.mark.parametrize("levels", [1, 2, 3, 4])
+def test_grid_builds(n, m, levels):
+    data = scenes.lidar_scene(n, seed=levels, extent=40.0)
+    q = np.ascontiguousarray(data[np.random.default_rng(m).permutation(n)[:m]] + np.float32(0.01))
+    _both(data, q, 12, grid_levels=levels)
+    rows = slice(0, 400)
+    oi, od = O.knn(data, q[rows], 12, kdtree=True)
+    with _Knobs(grid_levels=levels):
+        gi, gd = pgeof.knn_search(data, q, 12)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+
+
+def test_fused_row_offsets():
+    for n, k in ((1, 1), (63, 20), (4097, 108), (4097, 109)):
+        x = torch.from_numpy(scenes.uniform_cube(n, seed=n)).cuda()
+        k = min(k, n)
+        nn = torch.empty(n * k, dtype=torch.int32, device="cuda")
+        ptr = torch.full((n + 1,), -1, dtype=torch.int32, device="cuda")
+        f = torch.empty((n, 11), dtype=torch.float32, device="cuda")
+        capi.knn_features_device(x, k, nn, ptr, f)
+        np.testing.assert_array_equal(ptr.cpu().numpy(), np.arange(n + 1) * k)
+
+
 def test_queries_far_from_a_large_cloud():
     """Balls that grow from far outside the grid must not take the whole cloud
     at once (they would hold every point of it)."""
