@@ -38,10 +38,15 @@ __device__ __forceinline__ void features_of(const Moments& m, uint32_t k, float 
     features11(P, f);
 }
 
-// Neighbours gathered per chunk: the plain kernel's rows are short and its
+// Neighbours gathered per chunk.  The plain kernel's rows are short and its
 // per-neighbour work light, so it takes whole rows of up to 32 at once; the
-// multiscale and optimal kernels evaluate features or eigentropies inside
-// the loop and keep their registers for that (measured best: 32 and 8).
+// optimal kernel evaluates eigentropies inside the loop, one copy of that code
+// per neighbour of a chunk, and the multiscale kernel keeps its registers for
+// the features between the chunks.  Measured (ms per call; 3 M ragged rows,
+// mean 22 / 2 M rows of a radius of 64 at most with 4 scales and their search /
+// 1 M rows of 100 and theirs): plain 16 0.79, 28 0.73, 32 0.72, 40 1.43 (it
+// spills); multiscale 4 3.43, 8 3.12, 16 3.07, 24 3.50; optimal 4 2.77, 8 2.86.
+// More waves per SIMD by smaller chunks or spills are slower for all three.
 #ifndef PGEOF_CSR_CHUNK
 #define PGEOF_CSR_CHUNK 32
 #endif
@@ -49,7 +54,11 @@ __device__ __forceinline__ void features_of(const Moments& m, uint32_t k, float 
 #define PGEOF_CSR_WAVES_PER_SIMD 1
 #endif
 constexpr uint32_t kCsrChunkPlain = PGEOF_CSR_CHUNK;
-constexpr uint32_t kCsrChunkScales = 8;
+constexpr uint32_t kCsrChunkMulti = 16;
+constexpr uint32_t kCsrChunkOptimal = 4;
+
+// four indices at a 4-byte boundary
+typedef uint32_t Quad __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int MODE>
 __global__ __launch_bounds__(256, PGEOF_CSR_WAVES_PER_SIMD) void k_csr(CsrArgs a)
@@ -132,26 +141,36 @@ __global__ __launch_bounds__(256, PGEOF_CSR_WAVES_PER_SIMD) void k_csr(CsrArgs a
     // accumulated, so their loads overlap the gathers and the FP64 work
     // (10 M rows of 20: 5.5 ms with chunks of 4 and no look-ahead, 3.9 ms
     // with one chunk of 32).
-    constexpr uint32_t kChunk = MODE == kCsrPlain ? kCsrChunkPlain : kCsrChunkScales;
+    constexpr uint32_t kChunk = MODE == kCsrPlain ? kCsrChunkPlain : MODE == kCsrMulti ? kCsrChunkMulti : kCsrChunkOptimal;
     uint32_t nid[kChunk];
-    // a row that starts on a 16-byte boundary (every row of a kNN CSR with k
-    // a multiple of 4) is read four indices per load
-    const bool row16 = (reinterpret_cast<uintptr_t>(row) & 15u) == 0;
+    // Four indices per load, from any 4-byte boundary (a ragged CSR's rows
+    // start at all of them): one load per index touches a cache line per lane
+    // each time (3 M ragged rows of 22 on average, per call: 732 us with those
+    // for the rows off a 16-byte boundary, 722 now).  The last load of a row
+    // starts at its end - 4 and its entries move down.
     auto load_idx = [&](uint32_t j0) {
         static_assert(kChunk % 4 == 0, "chunks are read in groups of four");
 #pragma unroll
         for (uint32_t u = 0; u < kChunk; u += 4)
         {
-            uint32_t v[4];
-            if (row16 && j0 + u + 3 < walk)
+            const uint32_t at = j0 + u;
+            uint32_t v[4] = {i0, i0, i0, i0};
+            if (walk >= 4)
             {
-                const uint4 q = *reinterpret_cast<const uint4*>(row + j0 + u);
-                v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+                if (at < walk)
+                {
+                    const uint32_t from = min(at, walk - 4u);
+                    const Quad q = *reinterpret_cast<const Quad*>(row + from);
+                    const bool two = (at - from) & 2u, one = (at - from) & 1u;
+                    const uint32_t x = two ? q.z : q.x, y = two ? q.w : q.y, z = two ? i0 : q.z, w = two ? i0 : q.w;
+                    v[0] = one ? y : x, v[1] = one ? z : y, v[2] = one ? w : z, v[3] = one ? i0 : w;
+                }
             }
             else
             {
 #pragma unroll
-                for (uint32_t w = 0; w < 4; ++w) v[w] = (j0 + u + w < walk) ? row[j0 + u + w] : i0;
+                for (uint32_t w = 0; w < 3; ++w)
+                    if (at + w < walk) v[w] = row[at + w];
             }
 #pragma unroll
             for (uint32_t w = 0; w < 4; ++w)
@@ -162,7 +181,47 @@ __global__ __launch_bounds__(256, PGEOF_CSR_WAVES_PER_SIMD) void k_csr(CsrArgs a
         }
     };
     load_idx(0);
-    for (uint32_t j0 = 0; j0 < walk; j0 += kChunk)
+    if constexpr (MODE == kCsrMulti)
+    {
+        // One scale after the other, the same for every lane that has it: a
+        // chunk ends where a scale does, and the features stand in the code
+        // once (inside the loop over a chunk they stood there eight times,
+        // 73 KB of code, more than the instruction cache holds; 2 M rows of up to
+        // 64 with 4 scales 1.82 ms, now 1.1).
+        uint32_t j = 0;
+#pragma unroll 1
+        for (; s < a.n_scales; ++s)
+        {
+            const uint32_t scale = a.scales[s];
+            if (scale > walk) break;
+#pragma unroll 1
+            while (j < scale)
+            {
+                float px[kChunk], py[kChunk], pz[kChunk];
+                const uint32_t take = min(kChunk, scale - j);
+#pragma unroll
+                for (uint32_t u = 0; u < kChunk; ++u)
+                {
+                    if (u >= take) break;
+                    const float3 p = xyz3[nid[u]];
+                    px[u] = p.x;
+                    py[u] = p.y;
+                    pz[u] = p.z;
+                }
+                j += take;
+                if (j < walk) load_idx(j);
+#pragma unroll
+                for (uint32_t u = 0; u < kChunk; ++u)
+                {
+                    if (u >= take) break;
+                    mom_add(m, (double)px[u] - ox, (double)py[u] - oy, (double)pz[u] - oz);
+                }
+            }
+            features_of(m, scale, f);
+            store_row11(out + (size_t)s * 11, f);
+        }
+    }
+    for (uint32_t j0 = 0; MODE != kCsrMulti && j0 < walk; j0 += kChunk)
     {
         float px[kChunk], py[kChunk], pz[kChunk];
 #pragma unroll
@@ -180,16 +239,7 @@ __global__ __launch_bounds__(256, PGEOF_CSR_WAVES_PER_SIMD) void k_csr(CsrArgs a
             if (j0 + u >= walk) break;
             mom_add(m, (double)px[u] - ox, (double)py[u] - oy, (double)pz[u] - oz);
             const uint32_t cnt = j0 + u + 1;
-            if (MODE == kCsrMulti)
-            {
-                while (s < a.n_scales && a.scales[s] == cnt)
-                {
-                    features_of(m, cnt, f);
-                    store_row11(out + (size_t)s * 11, f);
-                    ++s;
-                }
-            }
-            else if (MODE == kCsrOptimal)
+            if (MODE == kCsrOptimal)
             {
                 if (cnt >= k0 && (cnt == k0 || cnt % a.k_step == 0 || cnt == k_nn))
                 {

@@ -278,3 +278,40 @@ def test_row_order_more_rows_than_points():
     ref = O.compute_features(data, nn, ptr)
     val = O.eigvals_csr_np(data, nn, ptr)
     assert_features_close(res[1][0], ref, val, "more rows than points")
+
+
+def test_rows_at_every_alignment():
+    """Rows of 0..70 neighbours starting at each 4-byte offset, all three
+    kernels, against the oracle and bit for bit whatever the row's offset."""
+    xyz = scenes.lidar_scene(5_000, seed=77, extent=8.0)
+    idx, _ = pgeof.knn_search(xyz, xyz, 70)
+    lens = np.arange(71)
+    sc = [2, 3, 4, 7, 16, 17, 32, 33, 50, 70]
+    got = []
+    for shift in range(4):
+        rows = [idx[0, :shift]] + [idx[100 + n, :n] for n in lens]
+        nn = np.concatenate(rows).astype(np.uint32)
+        ptr = np.r_[0, np.cumsum([len(r) for r in rows])].astype(np.uint32)
+        plain = pgeof.compute_features(xyz, nn, ptr)[1:]
+        multi = pgeof.compute_features_multiscale(xyz, nn, ptr, sc)[1:]
+        best = pgeof.compute_features_optimal(xyz, nn, ptr, 3, 2, 5)[1:]
+        got.append((plain, multi, best))
+    for g in got[1:]:
+        for a, b in zip(g, got[0]):
+            np.testing.assert_array_equal(a, b)
+    plain, multi, best = got[0]
+    nn = np.concatenate([idx[100 + n, :n] for n in lens]).astype(np.uint32)
+    ptr = np.r_[0, np.cumsum(lens)].astype(np.uint32)
+    assert_features_close(plain, O.compute_features(xyz, nn, ptr), O.eigvals_csr_np(xyz, nn, ptr), "plain")
+    # every scale is the plain row of that prefix, bit for bit (two or three
+    # points leave eigenvectors undefined: too few entries to compare with the
+    # oracle's)
+    for s, k in enumerate(sc):
+        pre = np.concatenate([idx[100 + n, :k] for n in range(k, 71)]).astype(np.uint32)
+        pptr = (np.arange(72 - k) * k).astype(np.uint32)
+        np.testing.assert_array_equal(multi[k:, s], pgeof.compute_features(xyz, pre, pptr))
+        assert (multi[:k, s] == 0).all()
+    ks = best[5:, 11].astype(int)
+    for n, k in zip(range(5, 71), ks):
+        row = pgeof.compute_features(xyz, nn[ptr[n] : ptr[n] + k].copy(), np.array([0, k], np.uint32))
+        np.testing.assert_array_equal(row[0], best[n, :11])
