@@ -499,7 +499,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
         const float4* __restrict__ pts = L->pts;
         const int cx = cell32(relx, ih, a0), cy = cell32(rely, ih, a1), cz = cell32(relz, ih, a2);
         const bool mine = (finite >> lane) & 1ull;
-        uint32_t around = 0;
+        uint32_t around = 0, rows = 0;  // points in the region, rows of cells that hold some
 #pragma unroll
         for (int r = 0; r < 9; ++r)
         {
@@ -507,7 +507,9 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
             if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
             {
                 const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
-                around += gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u) - gload(tcs, at + (uint32_t)max(cx - 1, 0));
+                const uint32_t c = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u) - gload(tcs, at + (uint32_t)max(cx - 1, 0));
+                around += c;
+                rows += c ? 1u : 0u;
             }
         }
         uint32_t inner, all;
@@ -564,6 +566,86 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
             wave_sync();
             write_rows(0, nq, kSparse, n);
             return;
+        }
+        // Up to 32 hits each: two lanes per query, 32 queries at a time, one
+        // lane filling a row from the front, the other from its end (200 k
+        // uniform points, 20 hits, cap 30: 241 us per call with a wave per query,
+        // 190 so; cap 64: 269, 203).
+        if (members <= 2)
+        {
+            // Points per row of cells up to which 32 hits are likely enough
+            // to try: 32 in the ball are 23 per row in a volume, 31 on a
+            // horizontal plane.  (224 per region whatever its rows: 1 M LiDAR
+            // points with 50 hits spent 64 us more on tries that failed.)
+            constexpr uint32_t kFewPair = 24;
+            constexpr uint32_t kPair = 2 * kPerLane, kPairStride = kPair + 1;
+            static_assert(32 * kPairStride <= sizeof(lds) / 8, "rows of the pairs");
+            const uint32_t odd = lane & 1u;
+            uint64_t* prow = lds + (lane >> 1) * kPairStride;
+            const uint32_t h0 = members == 2 ? wave & 1u : 0u, h1 = members == 2 ? h0 : 1u;
+            bool done = true;
+#pragma unroll 1
+            for (uint32_t half = h0; half <= h1 && 32 * half < nq; ++half)
+            {
+                const uint32_t ql = 32 * half + (lane >> 1);
+                const bool theirs = (finite >> ql) & 1ull;
+                done = __ballot(((lane >> 5) == half) && mine && (around > kFewPair * rows || inner < limit)) == 0;
+                if (!done) break;
+                const float x = __uint_as_float(from_lane(__float_as_uint(qv.x), ql)),
+                            y0 = __uint_as_float(from_lane(__float_as_uint(qv.y), ql)),
+                            z0 = __uint_as_float(from_lane(__float_as_uint(qv.z), ql));
+                const int px = (int)from_lane((uint32_t)cx, ql), py = (int)from_lane((uint32_t)cy, ql),
+                          pz = (int)from_lane((uint32_t)cz, ql);
+                uint32_t got = 0;
+#pragma unroll 1
+                for (int r = 0; r < 9; ++r)
+                {
+                    const int y = py + r % 3 - 1, z = pz + r / 3 - 1;
+                    uint32_t j = 0, e = 0;
+                    if (theirs && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
+                    {
+                        const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
+                        j = gload(tcs, at + (uint32_t)max(px - 1, 0)) + 4u * odd;
+                        e = gload(tcs, at + (uint32_t)min(px + 1, a0 - 1) + 1u);
+                    }
+                    for (; j < e; j += 8)
+                    {
+                        float4 p[4];
+#pragma unroll
+                        for (uint32_t u = 0; u < 4; ++u) p[u] = gload(pts, min(j + u, e - 1u));
+#pragma unroll
+                        for (uint32_t u = 0; u < 4; ++u)
+                        {
+                            const uint32_t d = min(__float_as_uint(sqdist32(x, y0, z0, p[u].x, p[u].y, p[u].z)), kNanBits);
+                            if (j + u < e && d <= limit)
+                            {
+                                if (got < kPair)
+                                    prow[odd ? kPair - 1 - got : got] = ((uint64_t)d << 32) | __float_as_uint(p[u].w);
+                                ++got;
+                            }
+                        }
+                    }
+                }
+                const uint32_t other = from_lane(got, lane ^ 1u), both = got + other;
+                done = __ballot(both > kPair) == 0;
+                if (!done) break;
+                wave_sync();
+                const uint32_t front = odd ? other : got, back = both - front;
+                double v[kPerLane];
+#pragma unroll
+                for (int r = 0; r < kPerLane; ++r)
+                {
+                    const uint32_t i = odd * kPerLane + (uint32_t)r;
+                    v[r] = __longlong_as_double((long long)(i < front || i >= kPair - back ? prow[i] : kNoKey));
+                }
+                sort_rows<2>(v, lane);
+#pragma unroll
+                for (int r = 0; r < kPerLane; ++r) prow[odd * kPerLane + r] = (uint64_t)__double_as_longlong(v[r]);
+                wave_sync();
+                write_rows(32 * half, min(32u, nq - 32 * half), kPairStride, from_lane(both, (2 * lane) & 63u));
+                wave_sync();
+            }
+            if (done) return;
         }
         if (members > 1)
         {

@@ -188,6 +188,21 @@ def test_radius_waves(n, hits):
     _radius_both(xyz, xyz, edge * float(np.cbrt(hits / (4.19 * n))), 30)
 
 
+# two lanes per query: 16 to 32 hits, caps below and above them, a last half
+# of 1, 31, 32 or 33 queries, one and two waves per 64 queries
+@pytest.mark.parametrize("n", [65_569, 65_599, 65_632, 65_633, 2_097_153])
+@pytest.mark.parametrize("hits,cap", [(14, 20), (20, 30), (20, 64), (24, 100), (30, 31)])
+def test_radius_pairs(n, hits, cap):
+    rng = np.random.default_rng(hits)
+    side = 40 if n < 1_000_000 else 127
+    at = np.stack(np.unravel_index(np.arange(n) % side**3, (side,) * 3), 1)  # jittered lattice: even density
+    xyz = (at + rng.uniform(-0.3, 0.3, (n, 3))).astype(np.float32)
+    xyz[n // 3 : n // 3 + 50] = xyz[5]  # and a spot of 50
+    data = xyz[rng.permutation(n)].copy()
+    density = n / side**3
+    _radius_both(data, data, float(np.cbrt(hits / (4.19 * density))), cap)
+
+
 @pytest.mark.parametrize("r", [0.0, 1e-30, np.inf, -0.5])
 def test_radius_values(r):
     xyz = scenes.uniform_cube(2000, seed=8)
