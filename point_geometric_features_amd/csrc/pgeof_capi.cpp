@@ -632,17 +632,16 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
 }
 
 // Whether a search takes the wave-per-query kernel: up to k (or cap) = 108,
-// the largest rows it keeps.  Faster than a lane per query with a heap at every
-// size and k measured (us per call, before -> now: 257 queries on 1,000
-// points at k = 10 228 -> 100; 10 k points at k = 20 227 -> 135; 100 k LiDAR
-// points at k = 20 1061 -> 430; 10 M 11.25 -> 7.9 ms; 4 M at k = 50
-// 13.2 -> 4.3 ms; 1 M at k = 100 7.1 -> 2.1 ms; radius r = 0.5, at most 64,
-// with features of 2 M points 6.9 -> 3.8 ms; r = 0.2, at most 30, 1 M sparse
-// points 384 -> 268 us).  Past 108 a row no longer
-// fits the lanes that sort it and the general search is the only one.
-// Radius searches of at most 16 stay with it: heaps that small live in
-// registers (1 M LiDAR points, r = 0.37, 50 in the ball: 0.70 ms against 0.81
-// for 16, but 1.34 against 0.82 for 30).
+// the largest rows it keeps; past that a row no longer fits the lanes that
+// sort it and the general search is the only one.  Faster than a lane per
+// query with a heap at every size and k measured, on the same grid build (us
+// per call, general -> wave: 1,000 points at k = 8 309 -> 79 LiDAR, 160 -> 63
+// uniform; 10 k at k = 16 664 -> 130, 185 -> 73; 200 k at k = 32 2366 -> 420,
+// 604 -> 233; 1 M at k = 64 5887 -> 1330, 3503 -> 1064), but for uniform
+// clouds of a million points at k = 4 (487 -> 548) where the two cross.
+// Radius searches of at most 16 stay with the heap, which at that size lives
+// in registers (1 M LiDAR points, r = 0.37, 50 in the ball: 0.70 ms against
+// 0.81 for 16, but 1.34 against 0.79 for 30).
 bool wave_path(uint32_t k, bool radius)
 {
     return k <= kWaveMaxK && (double)k <= tuning().wave_k_max && !(radius && k <= 16);

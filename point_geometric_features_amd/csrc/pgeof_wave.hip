@@ -20,7 +20,7 @@
 // (k_search, a lane per query with a heap, about 430, its lanes waiting for
 // each other: 3 times the candidate steps and 3.5 times the insertions of a
 // lane).  Search kernels per call, k_search -> this one: 10 M at k = 20 9.8 ->
-// 6.5 ms, 4 M at k = 50 12.5 -> 3.7 ms, 1 M uniform points at k = 50 2.6 ->
+// 6.0 ms, 4 M at k = 50 12.5 -> 3.7 ms, 1 M uniform points at k = 50 2.6 ->
 // 0.65 ms, 1 M at k = 100 7.1 -> 2.1 ms, 100 k at k = 20 1.8 -> 0.2 ms (there
 // single sparse queries held a lane for thousands of steps).
 #include <type_traits>
