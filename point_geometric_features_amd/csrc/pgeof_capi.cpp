@@ -639,12 +639,13 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
 // uniform; 10 k at k = 16 664 -> 130, 185 -> 73; 200 k at k = 32 2366 -> 420,
 // 604 -> 233; 1 M at k = 64 5887 -> 1330, 3503 -> 1064), but for uniform
 // clouds of a million points at k = 4 (487 -> 548) where the two cross.
-// Radius searches of at most 16 stay with the heap, which at that size lives
-// in registers (1 M LiDAR points, r = 0.37, 50 in the ball: 0.70 ms against
-// 0.81 for 16, but 1.34 against 0.79 for 30).
+// Radius searches of at most 21 stay with the heap, whose entries are all in
+// registers and LDS up to there (us per call, general / wave: 1 M LiDAR
+// points, 50 in the ball, cap 16 700 / 810, cap 30 1332 / 791; 300 k uniform
+// points, 17 in the ball, cap 18 184 / 211, cap 21 181 / 214, cap 40 259 / 209).
 bool wave_path(uint32_t k, bool radius)
 {
-    return k <= kWaveMaxK && (double)k <= tuning().wave_k_max && !(radius && k <= 16);
+    return k <= kWaveMaxK && (double)k <= tuning().wave_k_max && !(radius && k <= 21);
 }
 
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,

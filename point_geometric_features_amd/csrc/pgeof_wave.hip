@@ -1019,13 +1019,16 @@ hipError_t launch_wave_g(int mode, const WaveArgs& a, hipStream_t s)
 {
     const bool radius = mode == kModeRadius || mode == kModeRadiusCsr;
     const uint32_t nb = radius ? (a.n_query + 63) / 64 * (64 / a.q_per_wave) : (a.n_query + a.q_per_wave - 1) / a.q_per_wave;
-    switch (mode)
+    if (mode == kModeKnn)
+        k_wave_search<kModeKnn, G><<<nb, 64, 0, s>>>(a);
+    else if (mode == kModeKnnFeat)
+        k_wave_search<kModeKnnFeat, G><<<nb, 64, 0, s>>>(a);
+    else if constexpr (G >= 4)
     {
-        case kModeKnn: k_wave_search<kModeKnn, G><<<nb, 64, 0, s>>>(a); break;
-        case kModeKnnFeat: k_wave_search<kModeKnnFeat, G><<<nb, 64, 0, s>>>(a); break;
-        case kModeRadius: k_wave_search<kModeRadius, G><<<nb, 64, 0, s>>>(a); break;
-        case kModeRadiusCsr: k_wave_search<kModeRadiusCsr, G><<<nb, 64, 0, s>>>(a); break;
-        default: return hipErrorInvalidValue;
+        if (mode == kModeRadius)
+            k_wave_search<kModeRadius, G><<<nb, 64, 0, s>>>(a);
+        else
+            k_wave_search<kModeRadiusCsr, G><<<nb, 64, 0, s>>>(a);
     }
     return hipGetLastError();
 }
@@ -1042,8 +1045,12 @@ hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s)
     ProfScope ps(names[mode], s);
     // rows of up to 16 G kept candidates, at least about a fifth more than k:
     // a narrower margin takes more steps to find a threshold
-    if (a.k <= 12) return launch_wave_g<1>(mode, a, s);
-    if (a.k <= 27) return launch_wave_g<2>(mode, a, s);
+    // (radius searches hold a whole ball in their region, 12 groups of 64
+    // points rather than 6: 700 k uniform points, 63 hits, cap 24: 1034 us per
+    // call with G = 2)
+    const bool radius = mode & 1;
+    if (!radius && a.k <= 12) return launch_wave_g<1>(mode, a, s);
+    if (!radius && a.k <= 27) return launch_wave_g<2>(mode, a, s);
     if (a.k <= 54) return launch_wave_g<4>(mode, a, s);
     return launch_wave_g<8>(mode, a, s);
 }

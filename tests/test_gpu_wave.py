@@ -191,7 +191,7 @@ def test_radius_waves(n, hits):
 # two lanes per query: 16 to 32 hits, caps below and above them, a last half
 # of 1, 31, 32 or 33 queries, one and two waves per 64 queries
 @pytest.mark.parametrize("n", [65_569, 65_599, 65_632, 65_633, 2_097_153])
-@pytest.mark.parametrize("hits,cap", [(14, 20), (20, 30), (20, 64), (24, 100), (30, 31)])
+@pytest.mark.parametrize("hits,cap", [(14, 21), (14, 22), (20, 30), (20, 64), (24, 100), (30, 31)])
 def test_radius_pairs(n, hits, cap):
     rng = np.random.default_rng(hits)
     side = 40 if n < 1_000_000 else 127
