@@ -818,6 +818,8 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         if (is_radius)
             while (b.q_per_wave & (b.q_per_wave - 1)) b.q_per_wave &= b.q_per_wave - 1;
         b.margin = a.margin;
+        b.top_bit = 1;
+        while (b.top_bit <= (n - 1) / 2) b.top_bit *= 2;
         if (is_radius)
         {
             uint32_t bits;

@@ -129,6 +129,7 @@ struct WaveArgs
     uint32_t n_query;
     uint32_t k;
     uint32_t need;          // points the region of a query's level should hold (>= k)
+    uint32_t top_bit;       // highest bit of the largest point index
     uint32_t q_per_wave;    // consecutive queries per wave, 1..64 (radius: a power of two)
     float margin;           // slack of the cell faces, relative to h
     uint32_t limit;         // radius: largest float bits of a hit's squared distance, 0xFFFFFFFF: none can be one

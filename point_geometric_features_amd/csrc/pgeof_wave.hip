@@ -15,7 +15,7 @@
 // per lane.
 //
 // What bounds it: instruction issue and the latency of the few dependent
-// loads per region, at 13 waves per CU (LDS rows) and 12 (k > 27, registers):
+// loads per region, at 12 waves per CU (registers; the LDS rows allow 13):
 // 10 M LiDAR points at k = 20 take about 200 vector instructions per query
 // (k_search, a lane per query with a heap, about 430, its lanes waiting for
 // each other: 3 times the candidate steps and 3.5 times the insertions of a
@@ -128,6 +128,12 @@ __device__ __forceinline__ void order2(double& a, double& b)
     b = hi;
 }
 
+// a key as a double
+__device__ __forceinline__ double key_bits(uint32_t d, uint32_t id)
+{
+    return __longlong_as_double((long long)(((uint64_t)d << 32) | id));
+}
+
 template <int CTRL>
 __device__ __forceinline__ double dpp(double v)
 {
@@ -208,13 +214,15 @@ struct Candidates
 
     // A threshold tau with k <= n <= most candidates at or below it, first
     // tried at `guess`, by false position (counts grow about linearly with
-    // the squared distance on a surface), then by bisection of the bits.
+    // the squared distance on a surface), then in turns by the next distance
+    // above those that are too few, which settles ties, and by bisection of
+    // the bits, which bounds the steps.
     // Thresholds up to `closed` are preferred (no point outside the scanned
     // cells is nearer); past it open = true, and `outer` bounds all distances
     // that are expected.  No threshold passes `limit` (a radius search's):
     // with fewer than k candidates up to it tau = limit and n < k.  Ties at
-    // the k-th distance may leave no threshold: then n > most, and ties()
-    // bounds the indices.
+    // the k-th distance may leave no threshold: then n > most, tau is that
+    // distance, and ties() bounds the indices.
     __device__ __forceinline__ uint32_t select(uint32_t k, uint32_t most, uint32_t guess, uint32_t closed,
                                                uint32_t outer, uint32_t limit, uint32_t& n, bool& open) const
     {
@@ -251,6 +259,14 @@ struct Candidates
                 tau = (uint32_t)hi;
                 break;
             }
+            if (it >= 3 && (it & 1))
+            {
+                // no candidate lies between lo and the next one (if any)
+                const uint32_t top = hi_known ? (uint32_t)hi : cap, up = next_above(lo);
+                tau = up >= (uint32_t)(lo + 1) ? min(up, top) : top;
+                lo = (int)tau - 1;
+                continue;
+            }
             float next;
             if (hi_known)
             {
@@ -270,11 +286,9 @@ struct Candidates
         return tau < 0x7F800000u ? tau : min(tau, largest());
     }
 
-    __device__ __forceinline__ uint32_t largest() const
+    // of one value per lane
+    __device__ __forceinline__ static uint32_t wave_max(uint32_t m)
     {
-        uint32_t m = 0;
-#pragma unroll
-        for (int u = 0; u < NG; ++u) m = max(m, b[u] > kNanBits ? 0u : b[u]);
         m = max(m, dpp<kRowShr | 1>(m));
         m = max(m, dpp<kRowShr | 2>(m));
         m = max(m, dpp<kRowShr | 4>(m));
@@ -282,20 +296,50 @@ struct Candidates
         return max(max(readlane(m, 15u), readlane(m, 31u)), max(readlane(m, 47u), readlane(m, 63u)));
     }
 
-    // of the candidates exactly at tau, those with index <= the result make
-    // up k together with the nearer ones
-    __device__ __forceinline__ uint32_t ties(uint32_t k, uint32_t tau) const
+    __device__ __forceinline__ uint32_t largest() const
     {
-        const uint32_t want = k - (tau ? count(tau - 1u) : 0u);
-        uint32_t t = 0;
-        for (uint32_t bit = 0x80000000u; bit; bit >>= 1)
-        {
-            // largest t with fewer than `want` tied indices below it
-            uint32_t c = 0;
+        uint32_t m = 0;
 #pragma unroll
-            for (int u = 0; u < NG; ++u) c += (uint32_t)__popcll(__ballot(b[u] == tau && id[u] < (t | bit)));
-            if (c < want) t |= bit;
+        for (int u = 0; u < NG; ++u) m = max(m, b[u] > kNanBits ? 0u : b[u]);
+        return wave_max(m);
+    }
+
+    // the smallest distance bits above lo (>= -1); less than that if none are
+    __device__ __forceinline__ uint32_t next_above(int lo) const
+    {
+        uint32_t m = 0xFFFFFFFFu;
+#pragma unroll
+        for (int u = 0; u < NG; ++u) m = min(m, b[u] - (uint32_t)(lo + 1));  // those below wrap around
+        return ~wave_max(~m) + (uint32_t)(lo + 1);
+    }
+
+    // Of the candidates exactly at tau, those with index <= the result, with
+    // the nearer ones, are at least k and at most `most`: n.  By bisection of
+    // the indices from the highest bit of the largest one; any number in that
+    // range ends it (after about 5 steps; exactly k took all 32).
+    __device__ __forceinline__ uint32_t ties(uint32_t k, uint32_t most, uint32_t tau, uint32_t top_bit, uint32_t& n) const
+    {
+        const uint32_t nearer = tau ? count(tau - 1u) : 0u;
+        uint32_t tied[NG];
+#pragma unroll
+        for (int u = 0; u < NG; ++u) tied[u] = b[u] == tau ? id[u] : 0xFFFFFFFFu;
+        uint32_t t = 0;
+        for (uint32_t bit = top_bit;; bit >>= 1)
+        {
+            // t: fewer than k with the tied indices below it
+            uint32_t c = nearer;
+#pragma unroll
+            for (int u = 0; u < NG; ++u) c += (uint32_t)__popcll(__ballot(tied[u] < (t | bit)));
+            if (c < k)
+                t |= bit;
+            else if (c <= most)
+            {
+                n = c;
+                return (t | bit) - 1u;
+            }
+            if (bit <= 1u) break;
         }
+        n = k;
         return t;
     }
 
@@ -313,17 +357,21 @@ struct Candidates
             n += (uint32_t)__popcll(m);
         }
     }
-    // ... of a threshold and its n; returns the number kept
-    __device__ __forceinline__ uint32_t store(uint64_t* dst, uint32_t k, uint32_t most, uint32_t tau, uint32_t n) const
+    // ... of a threshold and its n; returns the number kept, and in `last` the
+    // largest index kept of those at the threshold
+    __device__ __forceinline__ uint32_t store(uint64_t* dst, uint32_t k, uint32_t most, uint32_t tau, uint32_t n,
+                                              uint32_t top_bit, uint32_t& last) const
     {
+        last = 0xFFFFFFFFu;
         if (n <= most)
         {
             store_if(dst, [&](uint32_t bb, uint32_t) { return bb <= tau; });
             return n;
         }
-        const uint32_t tie = ties(k, tau);
+        const uint32_t tie = ties(k, most, tau, top_bit, n);
         store_if(dst, [&](uint32_t bb, uint32_t i) { return bb < tau || (bb == tau && i <= tie); });
-        return k;
+        last = tie;
+        return n;
     }
 };
 
@@ -376,9 +424,14 @@ __device__ __forceinline__ uint32_t work_block(uint32_t b, uint32_t nb)
     return side ? nb - kRun - at * kRun + e : at * kRun + e;
 }
 
-// G: lanes that sort one query's row of kPerLane * G kept candidates
+// G: lanes that sort one query's row of kPerLane * G kept candidates.
+// Three waves per SIMD (168 registers): nothing spills but scalars, and the
+// LDS rows allow 13 waves per CU at most.  With four (128 registers, 5 to 9 of
+// them spilled for G <= 2): 10 M LiDAR points, k = 20, fused 7.75 ms instead
+// of 7.65, 300 k 486 us instead of 435, 1 M at k = 8 719 instead of 654; 1 M
+// uniform points at k = 20 602 instead of 616.
 template <int MODE, int G>
-__global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
+__global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
 {
     constexpr bool RADIUS = MODE == kModeRadius || MODE == kModeRadiusCsr;
     constexpr uint32_t kGroups = kGroupsOf<G>;
@@ -777,7 +830,8 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     tau = c.select(k, kMost, guess, readlane(closed, i), readlane(outer, i), limit, n, open);
                     bounded = tau < 0x7F800000u;
                     done = bounded && !open;
-                    if (done) n = c.store(row, k, kMost, tau, n);
+                    uint32_t tie;
+                    if (done) n = c.store(row, k, kMost, tau, n, a.top_bit, tie);
                 };
                 if (total <= 64u)
                     search(std::integral_constant<int, 1>{});
@@ -837,6 +891,9 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     st = gload(ucs, at + (uint32_t)xa);
                     len = gload(ucs, at + (uint32_t)xb + 1u) - st;
                 };
+                // of the points exactly at tau those with an index up to `tie`
+                // are collected
+                uint32_t tie = 0xFFFFFFFFu;
                 for (;;)
                 {
                     const float w = __uint_as_float(tau);
@@ -851,7 +908,11 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     uint32_t n_buf = 0;
                     bool again = false;
                     // the nearest of the collected keys stay (at least k, at
-                    // most kMost of them), tau drops to their threshold
+                    // most kMost of them), tau and tie drop to their bound.
+                    // (With the distance alone every further point of a spot
+                    // of coincident ones was collected again: 200 k LiDAR
+                    // points, 20 k of them at the origin, k = 20, 25.9 ms per
+                    // call; 3.7 now, the heaps of the general search 7.2.)
                     auto reduce = [&]() {
                         wave_sync();
                         Candidates<(int)kBufGroups> c;
@@ -866,7 +927,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                         uint32_t m;
                         const float t = __uint_as_float(tau) * target * __builtin_amdgcn_rcpf((float)n_buf);
                         tau = c.select(k, kMost, uniform(__float_as_uint(t)), kNanBits, kNanBits, kNanBits, m, open);
-                        n_buf = c.store(buf, k, kMost, tau, m);
+                        n_buf = c.store(buf, k, kMost, tau, m, a.top_bit, tie);
                     };
                     // one row of cells per lane, then the rows' points as one
                     // list spread over the lanes, kAhead groups loaded together
@@ -908,7 +969,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
 #pragma unroll
                             for (uint32_t u = 0; u < kAhead; ++u)
                             {
-                                const bool in = f0 + u * 64u + lane < tot && d[u] <= tau;
+                                const bool in = f0 + u * 64u + lane < tot && key_bits(d[u], id[u]) <= key_bits(tau, tie);
                                 const uint64_t m = __ballot(in);
                                 if (in) buf[n_buf + lanes_below(m)] = ((uint64_t)d[u] << 32) | id[u];
                                 n_buf += (uint32_t)__popcll(m);
@@ -933,6 +994,7 @@ __global__ __launch_bounds__(64, G <= 2 ? 4 : 3) void k_wave_search(WaveArgs a)
                     const double past = fmax(sqrt((double)w) - away, 0.25 * h) * f + away;
                     const uint32_t t = uniform(__float_as_uint((float)(past * past)));
                     tau = min(t < 0x7F800000u ? max(t, tau + 1u) : kNanBits, limit);
+                    tie = 0xFFFFFFFFu;
                 }
                 wave_sync();
                 for (uint32_t e = lane; e < n; e += 64) row[e] = buf[e];

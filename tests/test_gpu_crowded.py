@@ -1,0 +1,98 @@
+"""Crowded and tied clouds through the wave-per-query search (k <= 108).
+
+Spots of coincident points (a scanner's invalid returns at the origin, stacked
+scans), coordinates rounded to a lattice: many candidates at exactly the k-th
+distance.  The rows must be the oracle's (ties by index), and a call must not
+take longer than the general search (wave_k_max = 0), whose heaps reject a
+tied point by one compare.  Without an index in its bound the wave search took
+3.5 to 6.5 times as long on the clouds timed here, with it 0.6 to 1.0 times;
+the limit lies at 1.5.
+"""
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import point_geometric_features_amd as pgeof
+from oracle import oracle as O
+from point_geometric_features_amd import capi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+class _General:
+    """kNN and radius calls by the general search."""
+
+    def __enter__(self):
+        self.old = capi.get_tuning("wave_k_max")
+        capi.set_tuning("wave_k_max", 0)
+
+    def __exit__(self, *exc):
+        capi.set_tuning("wave_k_max", self.old)
+
+
+def _ms(call):
+    torch.cuda.synchronize()
+    t = time.perf_counter()
+    call()
+    torch.cuda.synchronize()
+    return (time.perf_counter() - t) * 1e3
+
+
+def _ratio(call):
+    """Time of the call over the general search's, in turns."""
+    wave, general = [], []
+    for _ in range(5):
+        wave.append(_ms(call))
+        with _General():
+            general.append(_ms(call))
+    print(f"wave {np.median(wave):.2f} ms, general {np.median(general):.2f} ms")
+    return np.median(wave[1:]) / np.median(general[1:])
+
+
+def _spot(n, spot, at=0.0):
+    xyz = scenes.lidar_scene(n, seed=41, extent=28.0)
+    xyz[np.random.default_rng(2).permutation(n)[:spot]] = at
+    return xyz
+
+
+def _crowded(name):
+    rng = np.random.default_rng(7)
+    if name == "origin":
+        return _spot(200_000, 20_000)
+    if name == "one_point":
+        return np.full((20_000, 3), 7.25, np.float32)
+    if name == "stacked":  # 500 places, 400 points each
+        return scenes.lidar_scene(500, seed=3, extent=2.0).repeat(400, 0)[rng.permutation(200_000)]
+    return np.round(scenes.lidar_scene(200_000, seed=9, extent=28.0) * 5) / np.float32(5)  # "rounded"
+
+
+@pytest.mark.parametrize("name", ["origin", "one_point", "stacked", "rounded"])
+@pytest.mark.parametrize("k", [1, 8, 12, 20, 27, 50, 108])
+def test_rows(name, k):
+    xyz = np.ascontiguousarray(_crowded(name))
+    rows = np.random.default_rng(k).choice(len(xyz), 60, replace=False)
+    spot = np.flatnonzero((xyz == xyz[(xyz == 0).all(1).argmax()]).all(1))[:8]
+    rows[: len(spot)] = spot  # some of a spot
+    q = np.ascontiguousarray(xyz[rows])
+    oi, od = O.knn(xyz, q, k, kdtree=False)
+    gi, gd = pgeof.knn_search(xyz, q, k)
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gd, od)
+    oi, od, _ = O.radius(xyz, q, 0.3, max(k, 22), kdtree=False)
+    gi, gd = pgeof.radius_search(xyz, q, 0.3, max(k, 22))
+    np.testing.assert_array_equal(gi, oi)
+    np.testing.assert_array_equal(gd, od)
+
+
+@pytest.mark.parametrize("name,k", [("origin", 8), ("origin", 50), ("one_point", 20)])
+def test_knn_time(name, k):
+    x = torch.from_numpy(np.ascontiguousarray(_crowded(name))).cuda()
+    assert _ratio(lambda: pgeof.knn_search(x, x, k)) < 1.5
+
+
+@pytest.mark.parametrize("name,r,cap", [("one_point", 0.3, 30)])
+def test_radius_time(name, r, cap):
+    x = torch.from_numpy(np.ascontiguousarray(_crowded(name))).cuda()
+    assert _ratio(lambda: pgeof.radius_search(x, x, r, cap)) < 1.5
