@@ -912,7 +912,7 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
                     // (With the distance alone every further point of a spot
                     // of coincident ones was collected again: 200 k LiDAR
                     // points, 20 k of them at the origin, k = 20, 25.9 ms per
-                    // call; 3.7 now, the heaps of the general search 7.2.)
+                    // call; 2.5 now, the heaps of the general search 7.2.)
                     auto reduce = [&]() {
                         wave_sync();
                         Candidates<(int)kBufGroups> c;
@@ -952,27 +952,46 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
                         const uint32_t tot = readlane(incl, 63u);
                         for (uint32_t f0 = 0; f0 < tot; f0 += 64 * kAhead)
                         {
-                            uint32_t d[kAhead], id[kAhead];
-#pragma unroll
-                            for (uint32_t u = 0; u < kAhead; ++u)
+                            uint32_t at[kAhead];
+                            // A candidate's row: the last one that starts at or
+                            // before it.  Where cells are crowded one row holds
+                            // all of them, found by two ballots instead of six
+                            // dependent LDS reads per candidate (100 k points
+                            // in a few cells, another far away, k = 50: 65.7 ->
+                            // 29.8 ms per call, 39.1 with a heap per lane).
+                            const uint32_t row0 = (uint32_t)__popcll(__ballot(first <= f0));
+                            if (row0 == (uint32_t)__popcll(__ballot(first < min(f0 + 64u * kAhead, tot))))
                             {
-                                // the last row that starts at or before candidate f
-                                const uint32_t f = min(f0 + u * 64u + lane, tot - 1u);
-                                uint32_t rw = 0;
+                                const uint32_t o = readlane(off, row0 - 1u);
 #pragma unroll
-                                for (uint32_t step = 32; step; step >>= 1)
-                                    rw = f >= from_lane(first, rw + step) ? rw + step : rw;
-                                const float4 p = gload(pts, f + from_lane(off, rw));
-                                d[u] = min(__float_as_uint(sqdist32(qxf, qyf, qzf, p.x, p.y, p.z)), kNanBits);
-                                id[u] = __float_as_uint(p.w);
+                                for (uint32_t u = 0; u < kAhead; ++u) at[u] = min(f0 + u * 64u + lane, tot - 1u) + o;
                             }
+                            else
+                            {
+#pragma unroll
+                                for (uint32_t u = 0; u < kAhead; ++u)
+                                {
+                                    const uint32_t f = min(f0 + u * 64u + lane, tot - 1u);
+                                    uint32_t rw = 0;
+#pragma unroll
+                                    for (uint32_t step = 32; step; step >>= 1)
+                                        rw = f >= from_lane(first, rw + step) ? rw + step : rw;
+                                    at[u] = f + from_lane(off, rw);
+                                }
+                            }
+                            float4 p[kAhead];
+#pragma unroll
+                            for (uint32_t u = 0; u < kAhead; ++u) p[u] = gload(pts, at[u]);
+                            __builtin_amdgcn_sched_barrier(0);  // (all of them before the first is used)
 #pragma unroll
                             for (uint32_t u = 0; u < kAhead; ++u)
                             {
-                                const bool in = f0 + u * 64u + lane < tot && key_bits(d[u], id[u]) <= key_bits(tau, tie);
+                                const uint32_t d = min(__float_as_uint(sqdist32(qxf, qyf, qzf, p[u].x, p[u].y, p[u].z)), kNanBits);
+                                const uint32_t id = __float_as_uint(p[u].w);
+                                const bool in = (f0 + u * 64u + lane < tot) & (key_bits(d, id) <= key_bits(tau, tie));
                                 const uint64_t m = __ballot(in);
-                                if (in) buf[n_buf + lanes_below(m)] = ((uint64_t)d[u] << 32) | id[u];
-                                n_buf += (uint32_t)__popcll(m);
+                                if (in) buf[n_buf + lanes_below(m)] = ((uint64_t)d << 32) | id;
+                                n_buf = uniform(n_buf + (uint32_t)__popcll(m));
                             }
                             if (n_buf > kBufKeys - 64u * kAhead)
                             {
