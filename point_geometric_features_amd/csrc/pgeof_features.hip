@@ -145,39 +145,53 @@ __global__ __launch_bounds__(256, PGEOF_CSR_WAVES_PER_SIMD) void k_csr(CsrArgs a
     uint32_t nid[kChunk];
     // Four indices per load, from any 4-byte boundary (a ragged CSR's rows
     // start at all of them): one load per index touches a cache line per lane
-    // each time (3 M ragged rows of 22 on average, per call: 732 us with those
-    // for the rows off a 16-byte boundary, 722 now).  The last load of a row
-    // starts at its end - 4 and its entries move down.
+    // each time.  The last load of a row starts at its end - 4 and its entries
+    // move down, except in waves whose rows all have a multiple of four (every
+    // kNN CSR of such a k): the shifts in every group cost the rows of 20 more
+    // than the loads save.  us per call, 10 M rows of 20 on a 16-byte boundary
+    // / off it / 4 M rows of 21 / 3 M ragged rows of 1 to 40: one load per
+    // index off the boundary 2222, 2696, 1070, 720; shifts in all groups 2376,
+    // 2438, 967, 717; this 2192, 2233, 963, 715.
+    const bool whole = __ballot(walk & 3u) == 0;
     auto load_idx = [&](uint32_t j0) {
         static_assert(kChunk % 4 == 0, "chunks are read in groups of four");
 #pragma unroll
-        for (uint32_t u = 0; u < kChunk; u += 4)
+        for (uint32_t u = 0; u < kChunk; ++u) nid[u] = i0;
+        if (whole)
         {
-            const uint32_t at = j0 + u;
-            uint32_t v[4] = {i0, i0, i0, i0};
-            if (walk >= 4)
-            {
-                if (at < walk)
-                {
-                    const uint32_t from = min(at, walk - 4u);
-                    const Quad q = *reinterpret_cast<const Quad*>(row + from);
-                    const bool two = (at - from) & 2u, one = (at - from) & 1u;
-                    const uint32_t x = two ? q.z : q.x, y = two ? q.w : q.y, z = two ? i0 : q.z, w = two ? i0 : q.w;
-                    v[0] = one ? y : x, v[1] = one ? z : y, v[2] = one ? w : z, v[3] = one ? i0 : w;
-                }
-            }
-            else
-            {
 #pragma unroll
-                for (uint32_t w = 0; w < 3; ++w)
-                    if (at + w < walk) v[w] = row[at + w];
-            }
-#pragma unroll
-            for (uint32_t w = 0; w < 4; ++w)
+            for (uint32_t u = 0; u < kChunk; u += 4)
             {
-                bad |= v[w] >= a.n_xyz;
-                nid[u + w] = v[w] < a.n_xyz ? v[w] : 0u;
+                if (j0 + u >= walk) break;
+                const Quad q = *reinterpret_cast<const Quad*>(row + j0 + u);
+                nid[u] = q.x, nid[u + 1] = q.y, nid[u + 2] = q.z, nid[u + 3] = q.w;
             }
+        }
+        else if (walk >= 4)
+        {
+#pragma unroll
+            for (uint32_t u = 0; u < kChunk; u += 4)
+            {
+                const uint32_t at = j0 + u;
+                if (at >= walk) break;
+                const uint32_t from = min(at, walk - 4u);
+                const Quad q = *reinterpret_cast<const Quad*>(row + from);
+                const bool two = (at - from) & 2u, one = (at - from) & 1u;
+                const uint32_t x = two ? q.z : q.x, y = two ? q.w : q.y, z = two ? i0 : q.z, w = two ? i0 : q.w;
+                nid[u] = one ? y : x, nid[u + 1] = one ? z : y, nid[u + 2] = one ? w : z, nid[u + 3] = one ? i0 : w;
+            }
+        }
+        else
+        {
+#pragma unroll
+            for (uint32_t w = 0; w < 3; ++w)
+                if (j0 + w < walk) nid[w] = row[j0 + w];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kChunk; ++u)
+        {
+            bad |= nid[u] >= a.n_xyz;
+            nid[u] = nid[u] < a.n_xyz ? nid[u] : 0u;
         }
     };
     load_idx(0);
