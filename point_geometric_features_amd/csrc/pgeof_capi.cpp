@@ -634,18 +634,24 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
 // Whether a search takes the wave-per-query kernel: up to k (or cap) = 108,
 // the largest rows it keeps; past that a row no longer fits the lanes that
 // sort it and the general search is the only one.  Faster than a lane per
-// query with a heap at every size and k measured, on the same grid build (us
-// per call, general -> wave: 1,000 points at k = 8 309 -> 79 LiDAR, 160 -> 63
-// uniform; 10 k at k = 16 664 -> 130, 185 -> 73; 200 k at k = 32 2366 -> 420,
-// 604 -> 233; 1 M at k = 64 5887 -> 1330, 3503 -> 1064), but for uniform
-// clouds of a million points at k = 4 (487 -> 548) where the two cross.
+// query with a heap at nearly every size and k measured, on the same grid
+// build (us per call, general -> wave: 1,000 points at k = 8 309 -> 79 LiDAR,
+// 160 -> 63 uniform; 10 k at k = 16 664 -> 130, 185 -> 73; 200 k at k = 32
+// 2366 -> 420, 604 -> 233; 1 M at k = 64 5887 -> 1330, 3503 -> 1064).
+// A cloud's search for the nearest point itself (k = 1, each point or one
+// with its coordinates) needs no heap and ends in its own cell: with a lane
+// per query from 2^16 points on (us per call, general / wave: 40 k points 130 /
+// 98 uniform, 149 / 139 LiDAR; 60 k 103 / 106, 143 / 173; 1 M 269 / 526, 349 /
+// 605; 10 M 2199 / 4663, 2838 / 4855).  Queries of their own keep the wave (1
+// M LiDAR points, 300 k queries around them: 14900 / 3310).
 // Radius searches of at most 21 stay with the heap, whose entries are all in
 // registers and LDS up to there (us per call, general / wave: 1 M LiDAR
 // points, 50 in the ball, cap 16 700 / 810, cap 30 1332 / 791; 300 k uniform
 // points, 17 in the ball, cap 18 184 / 211, cap 21 181 / 214, cap 40 259 / 209).
-bool wave_path(uint32_t k, bool radius)
+bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
 {
-    return k <= kWaveMaxK && (double)k <= tuning().wave_k_max && !(radius && k <= 21);
+    if (radius ? k <= 21 : (k == 1 && self && n >= (1u << 16))) return false;
+    return k <= kWaveMaxK && (double)k <= tuning().wave_k_max;
 }
 
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,
@@ -770,7 +776,8 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     a.n_scales = n_scales;
     const float4* qs = nullptr;
     const bool is_radius = mode == kModeRadius || mode == kModeRadiusCsr || mode == kModeRadiusMulti;
-    const bool wave = mode != kModeRadiusMulti && wave_path(k, is_radius);
+    const bool self = query == data && m == n;
+    const bool wave = mode != kModeRadiusMulti && wave_path(k, is_radius, self, n);
     int rc = build_grid(data, n, query, m, k, radius, is_radius, wave, w, a, &qs, s);
     if (rc) return rc;
     a.data = data;

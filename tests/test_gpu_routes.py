@@ -1,0 +1,76 @@
+"""Calls near the lines where a search goes over from the wave-per-query kernel
+to the general one: the same rows on both sides, and no side that the other
+would serve in much less time."""
+import time
+
+import numpy as np
+import pytest
+import torch
+
+import point_geometric_features_amd as pgeof
+from oracle import oracle as O
+from point_geometric_features_amd import capi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+class _General:
+    """kNN and radius calls by the general search."""
+
+    def __enter__(self):
+        self.old = capi.get_tuning("wave_k_max")
+        capi.set_tuning("wave_k_max", 0)
+
+    def __exit__(self, *exc):
+        capi.set_tuning("wave_k_max", self.old)
+
+
+def _ratio(call):
+    """Time of the call over the general search's, in turns."""
+
+    def ms():
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        for _ in range(3):
+            call()
+        torch.cuda.synchronize()
+        return (time.perf_counter() - t) * 1e3 / 3
+
+    ours, general = [], []
+    for _ in range(6):
+        ours.append(ms())
+        with _General():
+            general.append(ms())
+    print(f"{np.median(ours):.3f} ms, general {np.median(general):.3f} ms")
+    return np.median(ours[1:]) / np.median(general[1:])
+
+
+def _uniform(n, seed=3):
+    return torch.rand(n, 3, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda")
+
+
+@pytest.mark.parametrize("n", [65_535, 65_536])
+@pytest.mark.parametrize("own_queries", [False, True])
+def test_nearest_rows(n, own_queries):
+    """k = 1 around the line at 2^16 points, some of them twice."""
+    xyz = scenes.lidar_scene(n, seed=6, extent=16.0)
+    xyz[-50:] = xyz[:50]
+    q = xyz + np.float32(0.01) if own_queries else xyz
+    x = torch.from_numpy(xyz).cuda()
+    gi, gd = pgeof.knn_search(x, torch.from_numpy(q).cuda() if own_queries else x, 1)
+    gi, gd = gi.cpu().numpy(), gd.cpu().numpy()
+    rows = np.r_[0:60, n - 60:n]
+    oi, od = O.knn(xyz, np.ascontiguousarray(q[rows]), 1, kdtree=False)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+    if not own_queries:
+        same = np.arange(n)
+        same[-50:] = np.arange(50)
+        np.testing.assert_array_equal(gi[:, 0], same)
+
+
+def test_nearest_time():
+    """4 M uniform points, k = 1: by wave 1.9 times as long as the general
+    search, which they take; the limit lies at 1.3."""
+    x = _uniform(4_000_000)
+    assert _ratio(lambda: pgeof.knn_search(x, x, 1)) < 1.3
