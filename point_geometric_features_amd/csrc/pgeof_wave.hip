@@ -1125,12 +1125,15 @@ hipError_t launch_wave_search(int mode, const WaveArgs& a, hipStream_t s)
         return hipErrorInvalidValue;
     ProfScope ps(names[mode], s);
     // rows of up to 16 G kept candidates, at least about a fifth more than k:
-    // a narrower margin takes more steps to find a threshold
+    // a narrower margin takes more steps to find a threshold (k = 9, 10 and 12
+    // by G = 1 / 2, us per call: 10 M uniform points 4836, 5068, 5290 / 4619,
+    // 4721, 4711; 10 M LiDAR points 5640, 5755, 6059 / 5513, 5551, 5696; k = 8
+    // and fewer within 2 % either way)
     // (radius searches hold a whole ball in their region, 12 groups of 64
     // points rather than 6: 700 k uniform points, 63 hits, cap 24: 1034 us per
     // call with G = 2)
     const bool radius = mode & 1;
-    if (!radius && a.k <= 12) return launch_wave_g<1>(mode, a, s);
+    if (!radius && a.k <= 8) return launch_wave_g<1>(mode, a, s);
     if (!radius && a.k <= 27) return launch_wave_g<2>(mode, a, s);
     if (a.k <= 54) return launch_wave_g<4>(mode, a, s);
     return launch_wave_g<8>(mode, a, s);

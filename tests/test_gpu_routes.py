@@ -74,3 +74,26 @@ def test_nearest_time():
     search, which they take; the limit lies at 1.3."""
     x = _uniform(4_000_000)
     assert _ratio(lambda: pgeof.knn_search(x, x, 1)) < 1.3
+
+
+@pytest.mark.parametrize("k", [8, 9, 10, 12])
+@pytest.mark.parametrize("scene", ["lidar", "cube", "lattice"])
+def test_row_lengths(scene, k):
+    """Around k = 8, where the rows of kept candidates become longer."""
+    n = 20_011
+    xyz = scenes.lidar_scene(n, seed=8, extent=9.0) if scene == "lidar" else scenes.uniform_cube(n, seed=8)
+    if scene == "lattice":
+        xyz = np.floor(xyz * 20) / np.float32(20)
+    rows = np.r_[0:200, n - 200 : n]
+    oi, od = O.knn(xyz, np.ascontiguousarray(xyz[rows]), k, kdtree=False)
+    gi, gd = pgeof.knn_search(xyz, xyz, k)
+    np.testing.assert_array_equal(gi[rows], oi)
+    np.testing.assert_array_equal(gd[rows], od)
+    x = torch.from_numpy(xyz).cuda()
+    out = [torch.empty(n * k, dtype=torch.int32, device="cuda"), torch.empty(n + 1, dtype=torch.int32, device="cuda"),
+           torch.empty(n, 11, device="cuda")]
+    capi.knn_features_device(x, k, *out)
+    np.testing.assert_array_equal(out[0].cpu().numpy().reshape(n, k).astype(np.uint32), gi)
+    np.testing.assert_array_equal(out[1].cpu().numpy(), np.arange(n + 1) * k)
+    want = pgeof.compute_features(xyz, gi.reshape(-1), (np.arange(n + 1) * k).astype(np.uint32))
+    np.testing.assert_array_equal(out[2].cpu().numpy(), want)
