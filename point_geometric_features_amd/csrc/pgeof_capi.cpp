@@ -654,6 +654,19 @@ bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
     return k <= kWaveMaxK && (double)k <= tuning().wave_k_max;
 }
 
+// Whether the plan chooses between the two searches once it has seen how the
+// cloud fills its box: small k of large clouds searching themselves.  A wave
+// spends most of such a query on its region, a lane per query a step per
+// candidate, and what that loses is its lanes' uneven work: it loses little
+// where points lie evenly in a volume, and a wave much where cells at the
+// grid's cap hold points by the dozen (us per call, general / wave: uniform
+// points 1 M at k = 2 482 / 521, k = 8 573 / 540; 1.5 M 605 / 743, 726 / 781;
+// 10 M 3396 / 4649, 4048 / 4855, at k = 10 4307 / 4721, k = 12 4769 / 4711; 10
+// M LiDAR points 5447 / 4999, 8001 / 5509; a scanner's rings, 4 M points, 2669 /
+// 3822, 3782 / 4232, 2 M points 1737 / 2087, 2367 / 2286).  Both are queued, one
+// finds nothing to do: about 30 us, so not for smaller clouds.
+bool search_choice(uint32_t k, bool self, uint32_t n) { return self && k >= 2 && k <= 10 && n >= (5u << 18); }
+
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,
 // when query != data, sort the queries into level 0.  kNN sizes h_0 from the
 // target occupancy (k used for sizing); radius searches use one level with
@@ -662,7 +675,7 @@ bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
 // the kernels take their grid from the level table and the launches are
 // sized for the largest grid the workspace allows.
 int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, uint32_t k, float radius, bool is_radius,
-               bool wave, SearchWs& w, SearchArgs& sa, const float4** qs_out, hipStream_t s)
+               bool wave, bool choose, SearchWs& w, SearchArgs& sa, const float4** qs_out, hipStream_t s)
 {
     const Tuning t = tuning();
     const uint64_t cap = grid_cap(n);
@@ -672,6 +685,8 @@ int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, ui
     p.radius = radius;
     p.is_radius = is_radius ? 1 : 0;
     p.wave = wave ? 1 : 0;
+    p.choose = choose ? 1 : 0;
+    p.general_occupancy = t.knn_occupancy;
     p.cap = cap;
     // radius searches: one level, or for the wave-per-query search a second one
     // with half its cells' edge for the dense parts (2 M LiDAR points, r = 0.5,
@@ -778,7 +793,8 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
     const bool is_radius = mode == kModeRadius || mode == kModeRadiusCsr || mode == kModeRadiusMulti;
     const bool self = query == data && m == n;
     const bool wave = mode != kModeRadiusMulti && wave_path(k, is_radius, self, n);
-    int rc = build_grid(data, n, query, m, k, radius, is_radius, wave, w, a, &qs, s);
+    const bool choose = wave && !is_radius && search_choice(k, self, n);
+    int rc = build_grid(data, n, query, m, k, radius, is_radius, wave, choose, w, a, &qs, s);
     if (rc) return rc;
     a.data = data;
     a.queries = qs;
@@ -824,6 +840,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, std::max(std::min<uint32_t>(32u, m / 2048), m / 32768)));
         if (is_radius)
             while (b.q_per_wave & (b.q_per_wave - 1)) b.q_per_wave &= b.q_per_wave - 1;
+        b.other = choose ? &w.tab->count[0] : nullptr;
         b.margin = a.margin;
         b.top_bit = 1;
         while (b.top_bit <= (n - 1) / 2) b.top_bit *= 2;
@@ -841,7 +858,8 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         b.out_ptr = out_ptr;
         HIP_TRY(launch_wave_search(mode, b, s));
     }
-    else if (mode == kModeKnn || mode == kModeKnnFeat)
+    const bool general = !wave || choose;
+    if (general && (mode == kModeKnn || mode == kModeKnnFeat))
     {
         // Budgeted passes, finest level first: a query whose k-th neighbour
         // lies beyond +-2 cells of the level is flagged and, compacted and in
@@ -855,7 +873,7 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         // queries and take their count from it.
         const float4* list = qs;
         const float* blist = nullptr;
-        const uint64_t* n_dev = nullptr;  // queries in `list` (nullptr: all m)
+        const uint64_t* n_dev = choose ? &w.tab->count[0] : nullptr;  // queries in `list` (nullptr: all m)
         float4* next = w.qlist;
         float* bnext = w.blist;
         const int max_levels = std::max(1, std::min(kMaxLevels, (int)tuning().grid_levels));
@@ -895,9 +913,9 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         b.defer_bound = nullptr;
         HIP_TRY(launch_search(mode, b, hp.block, hp.lds, hp.global, false, s));
     }
-    else
+    else if (general)
         HIP_TRY(launch_search(mode, a, hp.block, hp.lds, hp.global, false, s));
-    if (out_ptr && !wave) HIP_TRY(launch_arange_ptr(out_ptr, m, k, s));
+    if (out_ptr && general) HIP_TRY(launch_arange_ptr(out_ptr, m, k, s));
     if (ws_out) *ws_out = w;
     return PGEOF_OK;
 }
@@ -1086,7 +1104,7 @@ int selected_host(const T* xyz, int64_t n, T search_radius, uint32_t max_knn, co
     if (wa.off > wa.size) return fail(PGEOF_ENOMEM, "workspace too small");
     SearchArgs sa{};
     const float4* qs = nullptr;
-    rc = build_grid(d_xf, (uint32_t)n, d_xf, (uint32_t)n, cap, (float)search_radius, true, false, w, sa, &qs, s);
+    rc = build_grid(d_xf, (uint32_t)n, d_xf, (uint32_t)n, cap, (float)search_radius, true, false, false, w, sa, &qs, s);
     if (rc) return rc;
     // this host entry point synchronises anyway: the kernel takes level 0 by value
     LevelTable tab;

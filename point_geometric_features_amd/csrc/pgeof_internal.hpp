@@ -66,7 +66,9 @@ struct LevelTable
     float bb[8];             // bounding box of the finite data coordinates: lo xyz, hi xyz
     unsigned long long sumsq;  // probe: sum of squared cell counts
     double hcap, T, h1;      // planning intermediates (grid-size floor, target occupancy, first guess)
-    uint64_t count[kMaxLevels + 2];  // kNN: queries left after each budgeted pass (device-side work counters)
+    // kNN: queries of the general search (count[0], where the plan chooses between
+    // it and the wave search) and those left after each budgeted pass
+    uint64_t count[kMaxLevels + 2];
 };
 
 // Everything the planning kernels need to size the grids of a search.
@@ -77,6 +79,8 @@ struct PlanArgs
     float radius;
     int is_radius;
     int wave;        // radius: levels for the wave-per-query search
+    int choose;      // kNN: the plan chooses the search (tab->count[0] = n: the general one, 0: by wave)
+    double general_occupancy;  // knn_occupancy of the general search
     uint64_t cap;  // largest G of level 0 (grid_cells_per_point * n)
     int max_levels;
     double knn_occupancy, knn_cell_points_max, radius_cell_factor, level_ratio;
@@ -131,6 +135,7 @@ struct WaveArgs
     uint32_t need;          // points the region of a query's level should hold (>= k)
     uint32_t top_bit;       // highest bit of the largest point index
     uint32_t q_per_wave;    // consecutive queries per wave, 1..64 (radius: a power of two)
+    const uint64_t* other;  // nothing to do where this is not 0 (the general search's queries), or nullptr
     float margin;           // slack of the cell faces, relative to h
     uint32_t limit;         // radius: largest float bits of a hit's squared distance, 0xFFFFFFFF: none can be one
     float r2;               // radius: search_radius * search_radius

@@ -447,7 +447,27 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         h = h1;
         if (m1 > T) h = h1 * sqrt(T / m1);
         h = fmax(h, hcap);
+        if (p.choose)
+        {
+            // The general search takes clouds that fill a volume evenly (its
+            // lanes have the same work, hardly a query is deferred), with its
+            // own smaller cells, and those whose points crowd in cells at the
+            // cap (candidates by the hundred for a few neighbours, at
+            // 400 k points per neighbour); see search_choice().
+            const bool even = m1 <= 2.0 * T;
+            const bool crowded = m1 * (h / h1) * (h / h1) > 30.0 && (double)p.n >= 4e5 * (double)p.k;
+            if (even)
+            {
+                const double Tg = fmax(0.75, fmin(p.general_occupancy * (double)p.k, p.knn_cell_points_max));
+                const double mg = 1.0 + (m1 - 1.0) * Tg / T;
+                h = h1 * cbrt(Tg / T);
+                if (mg > Tg) h *= sqrt(Tg / mg);
+                h = fmax(h, hcap);
+            }
+            tab->count[0] = even || crowded ? p.n : 0;
+        }
     }
+    if (p.choose && !(emax > 0.0)) tab->count[0] = 0;
     int nl = 0;
     for (int l = 0; l < levels; ++l)
     {
@@ -2500,11 +2520,14 @@ __global__ __launch_bounds__(256) void k_bound_scatter(const float4* __restrict_
                                                        const uint32_t* __restrict__ start, float4* __restrict__ q_out,
                                                        float* __restrict__ bound_out)
 {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= dyn_count(n_max, n_dev, 0)) return;
-    const uint32_t p = start[key[i]] + rank[i];
-    q_out[p] = q[i];
-    bound_out[p] = bound[i];
+    // (a launch sized for all queries leaves few blocks without work)
+    const uint64_t n = dyn_count(n_max, n_dev, 0);
+    for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u)
+    {
+        const uint32_t p = start[key[i]] + rank[i];
+        q_out[p] = q[i];
+        bound_out[p] = bound[i];
+    }
 }
 
 hipError_t launch_order_by_bound(const float4* q, const float* bound, uint32_t n_max, const uint64_t* n_dev,
@@ -2518,7 +2541,7 @@ hipError_t launch_order_by_bound(const float4* q, const float* bound, uint32_t n
     k_bound_hist<<<(n_max + 256 * 16 - 1) / (256 * 16), 256, 0, s>>>(bound, n_max, n_dev, count, key, rank);
     e = launch_scan_exclusive(count, count, kBoundBuckets + 1, scan_part, s);
     if (e != hipSuccess) return e;
-    k_bound_scatter<<<(n_max + 255) / 256, 256, 0, s>>>(q, bound, n_max, n_dev, key, rank, count, q_out, bound_out);
+    k_bound_scatter<<<blocks_for(n_max, 256, 4096), 256, 0, s>>>(q, bound, n_max, n_dev, key, rank, count, q_out, bound_out);
     return hipGetLastError();
 }
 

@@ -434,6 +434,7 @@ template <int MODE, int G>
 __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
 {
     constexpr bool RADIUS = MODE == kModeRadius || MODE == kModeRadiusCsr;
+    if (!RADIUS && a.other && *a.other) return;
     constexpr uint32_t kGroups = kGroupsOf<G>;
     constexpr uint32_t kMost = (uint32_t)(kPerLane * G);  // candidates kept per query
     constexpr uint32_t kBatch = 64 / G;                   // queries collected before their rows are sorted

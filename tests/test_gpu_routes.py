@@ -97,3 +97,61 @@ def test_row_lengths(scene, k):
     np.testing.assert_array_equal(out[1].cpu().numpy(), np.arange(n + 1) * k)
     want = pgeof.compute_features(xyz, gi.reshape(-1), (np.arange(n + 1) * k).astype(np.uint32))
     np.testing.assert_array_equal(out[2].cpu().numpy(), want)
+
+
+def _rings(n, seed=4):
+    """A scanner's rings on the ground, turn after turn 1 m further: crowded
+    cells near the scanner, sparse ones far out."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    cols = n // 64
+    c = torch.arange(cols, device="cuda", dtype=torch.float64)
+    az, turn = (c % 2048) * (2 * np.pi / 2048), torch.floor(c / 2048)
+    el = torch.linspace(-0.43, -0.03, 64, device="cuda", dtype=torch.float64)
+    r = 1.8 / torch.tan(-el)[None, :] + 0.02 * torch.randn(cols, 64, generator=g, device="cuda", dtype=torch.float64)
+    xyz = torch.stack([r * torch.cos(az)[:, None] + turn[:, None], r * torch.sin(az)[:, None],
+                       -r * torch.tan(-el)[None, :]], -1)
+    return xyz.reshape(-1, 3).float().contiguous()
+
+
+@pytest.mark.parametrize("n", [(5 << 18) - 1, 5 << 18])
+@pytest.mark.parametrize("k", [2, 5, 10, 11])
+@pytest.mark.parametrize("scene", ["uniform", "lidar", "rings", "one_point", "not_finite"])
+def test_chosen_rows(scene, n, k):
+    """From 1,310,720 points on (k = 2 to 10) the plan chooses the search."""
+    x = _rings((n + 63) // 64 * 64)[:n].contiguous() if scene == "rings" else _uniform(n)
+    if scene == "lidar":
+        x = torch.from_numpy(scenes.lidar_scene(n, seed=11, extent=72.0)).cuda()
+    elif scene == "one_point":
+        if k != 2:
+            pytest.skip("the same at every k")
+        x[1000:] = x[0]
+        x = x[: 40_000].contiguous()
+        n = len(x)
+    elif scene == "not_finite":
+        x[5] = float("nan")
+        x[n - 1, 2] = float("inf")
+    rows = np.r_[0:20, n - 20 : n]
+    xyz = x.cpu().numpy()
+    gi, gd = pgeof.knn_search(x, x, k)
+    if scene != "not_finite":  # (the oracle's scan does not order NaN distances)
+        oi, od = O.knn(xyz, np.ascontiguousarray(xyz[rows]), k, kdtree=False)
+        np.testing.assert_array_equal(gi.cpu().numpy()[rows], oi)
+        np.testing.assert_array_equal(gd.cpu().numpy()[rows], od)
+    out = [torch.empty(n * k, dtype=torch.int32, device="cuda"), torch.empty(n + 1, dtype=torch.int32, device="cuda"),
+           torch.empty(n, 11, device="cuda")]
+    capi.knn_features_device(x, k, *out)
+    with _General():
+        wi, wd = pgeof.knn_search(x, x, k)
+        want = [torch.empty_like(o) for o in out]
+        capi.knn_features_device(x, k, *want)
+    assert torch.equal(gi.view(torch.int32), wi.view(torch.int32)) and torch.equal(gd, wd)
+    assert torch.equal(out[0], want[0]) and torch.equal(out[1], want[1])
+    assert torch.equal(out[2].view(torch.int32), want[2].view(torch.int32))
+
+
+@pytest.mark.parametrize("cloud,k,limit", [(_uniform, 2, 1.15), (_uniform, 4, 1.15), (_rings, 2, 1.15)])
+def test_chosen_time(cloud, k, limit):
+    """4 M points: by wave 1.26 to 1.4 times as long as the general search, by
+    the plan's choice within a few per cent of it."""
+    x = cloud(1 << 22)
+    assert _ratio(lambda: pgeof.knn_search(x, x, k)) < limit
