@@ -648,6 +648,12 @@ void level_tables(uint32_t* cs_all, uint64_t cap, uint32_t* cs[kMaxLevels], uint
 // registers and LDS up to there (us per call, general / wave: 1 M LiDAR
 // points, 50 in the ball, cap 16 700 / 810, cap 30 1332 / 791; 300 k uniform
 // points, 17 in the ball, cap 18 184 / 211, cap 21 181 / 214, cap 40 259 / 209).
+// Above 21 the wave is ahead on LiDAR scenes from 5 hits on and everywhere from
+// cap 50 on; below cap 32 it is behind where hits are fewer than that (1 M LiDAR
+// points, r = 0.05, cap 22 320 / 371, cap 30 377 / 379) and in evenly filled
+// volumes of 1 M points and more with 20 to 130 hits (1 M, 34 hits, cap 22
+// 631 / 813, cap 30 809 / 815; 2 M, 28 hits, cap 24 1161 / 1540, cap 40 1462 /
+// 1569; 2 M, 131 hits, cap 30 2276 / 2698): neither shows on the host.
 bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
 {
     if (radius ? k <= 21 : (k == 1 && self && n >= (1u << 16))) return false;

@@ -511,25 +511,44 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
     // Sorted rows of the queries first .. first + count, `stride` keys apart
     // in LDS; lane s holds the number of keys of query first + s.
     auto write_rows = [&](uint32_t first, uint32_t count, uint32_t stride, uint32_t keys) {
-#pragma unroll 4
-        for (uint32_t s = 0; s < count; ++s)
+        auto store_key = [&](uint32_t* oi, float* od, uint32_t e, uint64_t key, uint32_t hits) {
+            const bool none = RADIUS ? e >= hits : key == kNoKey;
+            oi[e] = none ? 0xFFFFFFFFu : (uint32_t)key;
+            // past the hits 0, and r^2 in the last slot (nanoflann's
+            // RKNNResultSet::init)
+            const float pad = !RADIUS ? INFINITY : (e == k - 1 ? a.r2 : 0.0f);
+            if (od) od[e] = none ? pad : __uint_as_float((uint32_t)(key >> 32));
+        };
+        if (RADIUS && k <= 32)
         {
-            const uint32_t qorig = readlane(__float_as_uint(qv.w), first + s);
-            uint32_t* oi = a.out_idx + (size_t)qorig * k;
-            float* od = a.out_d2 ? a.out_d2 + (size_t)qorig * k : nullptr;
-            const uint32_t hits = RADIUS ? min(readlane(keys, s), k) : k;
-#pragma unroll
-            for (uint32_t e0 = 0; e0 < kMost; e0 += 64)
+            // two rows per store, one per half of the wave
+            const uint32_t e = lane & 31u;
+#pragma unroll 4
+            for (uint32_t s = lane >> 5; s < ((count + 1) & ~1u); s += 2)
             {
-                const uint32_t e = e0 + lane;
-                if (e >= (MODE == kModeRadiusCsr ? hits : k)) continue;
-                const uint64_t key = lds[s * stride + min(e, stride - 1u)];
-                const bool none = RADIUS ? e >= hits : key == kNoKey;
-                oi[e] = none ? 0xFFFFFFFFu : (uint32_t)key;
-                // past the hits 0, and r^2 in the last slot (nanoflann's
-                // RKNNResultSet::init)
-                const float pad = !RADIUS ? INFINITY : (e == k - 1 ? a.r2 : 0.0f);
-                if (od) od[e] = none ? pad : __uint_as_float((uint32_t)(key >> 32));
+                const uint32_t qorig = from_lane(__float_as_uint(qv.w), (first + s) & 63u);
+                const uint32_t hits = min(from_lane(keys, s & 63u), k);
+                if (s < count && e < (MODE == kModeRadiusCsr ? hits : k))
+                    store_key(a.out_idx + (size_t)qorig * k, a.out_d2 ? a.out_d2 + (size_t)qorig * k : nullptr, e,
+                              lds[s * stride + min(e, stride - 1u)], hits);
+            }
+        }
+        else
+        {
+#pragma unroll 4
+            for (uint32_t s = 0; s < count; ++s)
+            {
+                const uint32_t qorig = readlane(__float_as_uint(qv.w), first + s);
+                uint32_t* oi = a.out_idx + (size_t)qorig * k;
+                float* od = a.out_d2 ? a.out_d2 + (size_t)qorig * k : nullptr;
+                const uint32_t hits = RADIUS ? min(readlane(keys, s), k) : k;
+#pragma unroll
+                for (uint32_t e0 = 0; e0 < kMost; e0 += 64)
+                {
+                    const uint32_t e = e0 + lane;
+                    if (e >= (MODE == kModeRadiusCsr ? hits : k)) continue;
+                    store_key(oi, od, e, lds[s * stride + min(e, stride - 1u)], hits);
+                }
             }
         }
         if (RADIUS && a.out_count)
@@ -553,40 +572,79 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
         const float4* __restrict__ pts = L->pts;
         const int cx = cell32(relx, ih, a0), cy = cell32(rely, ih, a1), cz = cell32(relz, ih, a2);
         const bool mine = (finite >> lane) & 1ull;
-        uint32_t around = 0, rows = 0;  // points in the region, rows of cells that hold some
-#pragma unroll
-        for (int r = 0; r < 9; ++r)
+        // The part of the 27 cells that the ball can meet: where the cap of the
+        // grid makes its cells larger than the radius, about two of the nine
+        // rows (1 M uniform points, r = 0.2, cap 30: 352 us per call with all
+        // nine, 279 now; 1 M LiDAR points, r = 0.02, cap 24: 438, 307).
+        const float reach = sqrtf(__uint_as_float(min(limit, 0x7F800000u))) * 1.00001f;
+        int x0 = max(cx - 1, 0), x1 = min(cx + 1, a0 - 1), y0 = max(cy - 1, 0), y1 = min(cy + 1, a1 - 1),
+            z0 = max(cz - 1, 0), z1 = min(cz + 1, a2 - 1);
+        if (h > 1.25f * reach)
         {
-            const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
-            if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
+            const float w = reach + slack + h * a.margin;
+            x0 = max(x0, cell32(relx - w, ih, a0)), x1 = min(x1, cell32(relx + w, ih, a0));
+            y0 = max(y0, cell32(rely - w, ih, a1)), y1 = min(y1, cell32(rely + w, ih, a1));
+            z0 = max(z0, cell32(relz - w, ih, a2)), z1 = min(z1, cell32(relz + w, ih, a2));
+        }
+        const int ny = y1 - y0 + 1, n_rows = mine ? ny * (z1 - z0 + 1) : 0;
+        // the first cell of the rows one after the other, ny per layer
+        struct Rows
+        {
+            uint32_t at, step, skip;
+            int y, ny;
+            __device__ __forceinline__ void next()
             {
-                const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
-                const uint32_t c = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u) - gload(tcs, at + (uint32_t)max(cx - 1, 0));
+                at += step;
+                if (++y == ny) y = 0, at += skip;
+            }
+        };
+        auto rows_from = [&](uint32_t first, int n) {
+            return Rows{first, (uint32_t)a0, (uint32_t)(a1 - n) * (uint32_t)a0, 0, n};
+        };
+        const uint32_t first_row = ((uint32_t)z0 * (uint32_t)a1 + (uint32_t)y0) * (uint32_t)a0;
+        uint32_t around = 0, rows = 0;  // points in them, rows that hold some
+        Rows R = rows_from(first_row, ny);
+#pragma unroll
+        for (int r = 0; r < 9; ++r, R.next())
+        {
+            if (__ballot(r < n_rows) == 0) break;
+            if (r < n_rows)
+            {
+                const uint32_t c = gload(tcs, R.at + (uint32_t)x1 + 1u) - gload(tcs, R.at + (uint32_t)x0);
                 around += c;
                 rows += c ? 1u : 0u;
             }
         }
         uint32_t inner, all;
         cover(cx, cy, cz, h, a0, a1, a2, inner, all);
-        // (no more than 16 around any: no more hits, the first wave's work)
-        if (wave % members && __ballot(mine && (around > (uint32_t)kPerLane || inner < limit)) == 0) return;
+        // No more than 16 around any: no more hits, the first wave's work.
+        // Else each wave of the group looks at its own queries, q0 .. q0 + n_own
+        // (all 64 scanned by each, the first to write them: 2 M uniform points
+        // with 8 hits, cap 24, 895 us, now 847).
+        const bool alone = members == 1 || __ballot(mine && (around > (uint32_t)kPerLane || inner < limit)) == 0;
+        if (alone && wave % members) return;
+        const uint32_t q0 = alone ? 0u : wave % members * a.q_per_wave;
+        if (q0 >= nq) return;
+        const uint32_t n_own = alone ? nq : min(a.q_per_wave, nq - q0);
+        const bool own = mine && lane - q0 < n_own;
         constexpr uint32_t kFew = 80;  // points a lane looks at
         uint32_t n = 0;
         constexpr uint32_t kSparse = (uint32_t)kPerLane + 1;
         static_assert(64 * kSparse <= sizeof(lds) / 8, "rows of the sparse case");
-        uint64_t* row = lds + lane * kSparse;
-        if (__ballot(mine && (around > kFew || inner < limit)) == 0)
+        uint64_t* row = lds + ((lane - q0) & 63u) * kSparse;
+        const int own_rows = own ? n_rows : 0;
+        if (__ballot(own && (around > kFew || inner < limit)) == 0)
         {
+            Rows S = rows_from(first_row, ny);
 #pragma unroll 1
-            for (int r = 0; r < 9; ++r)
+            for (int r = 0; r < 9; ++r, S.next())
             {
-                const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+                if (__ballot(r < own_rows) == 0) break;
                 uint32_t j = 0, e = 0;
-                if (mine && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
+                if (r < own_rows)
                 {
-                    const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
-                    j = gload(tcs, at + (uint32_t)max(cx - 1, 0));
-                    e = gload(tcs, at + (uint32_t)min(cx + 1, a0 - 1) + 1u);
+                    j = gload(tcs, S.at + (uint32_t)x0);
+                    e = gload(tcs, S.at + (uint32_t)x1 + 1u);
                 }
                 for (; j < e; j += 4)
                 {
@@ -608,9 +666,8 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
         }
         else
             n = (uint32_t)kPerLane + 1u;
-        if (__ballot(mine && n > (uint32_t)kPerLane) == 0)
+        if (__ballot(own && n > (uint32_t)kPerLane) == 0)
         {
-            if (wave % members) return;
             double v[kPerLane];
 #pragma unroll
             for (int r = 0; r < kPerLane; ++r) v[r] = __longlong_as_double((long long)((uint32_t)r < n ? row[r] : kNoKey));
@@ -618,7 +675,7 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
 #pragma unroll
             for (int r = 0; r < kPerLane; ++r) row[r] = (uint64_t)__double_as_longlong(v[r]);
             wave_sync();
-            write_rows(0, nq, kSparse, n);
+            write_rows(q0, n_own, kSparse, from_lane(n, (lane + q0) & 63u));
             return;
         }
         // Up to 32 hits each: two lanes per query, 32 queries at a time, one
@@ -629,38 +686,40 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
         {
             // Points per row of cells up to which 32 hits are likely enough
             // to try: 32 in the ball are 23 per row in a volume, 31 on a
-            // horizontal plane.  (224 per region whatever its rows: 1 M LiDAR
-            // points with 50 hits spent 64 us more on tries that failed.)
-            constexpr uint32_t kFewPair = 24;
+            // horizontal plane; in a volume one of 32 queries is past them
+            // from 22 hits on average, 16 per row.  (224 per region whatever
+            // its rows: 1 M LiDAR points with 50 hits spent 64 us more on tries
+            // that failed; 24 per row in a volume too: 2 M uniform points with
+            // 28 hits 1813 us, now 1550.)
+            constexpr uint32_t kFewPair = 24, kFewVolume = 18;
             constexpr uint32_t kPair = 2 * kPerLane, kPairStride = kPair + 1;
             static_assert(32 * kPairStride <= sizeof(lds) / 8, "rows of the pairs");
             const uint32_t odd = lane & 1u;
             uint64_t* prow = lds + (lane >> 1) * kPairStride;
-            const uint32_t h0 = members == 2 ? wave & 1u : 0u, h1 = members == 2 ? h0 : 1u;
             bool done = true;
 #pragma unroll 1
-            for (uint32_t half = h0; half <= h1 && 32 * half < nq; ++half)
+            for (uint32_t first = q0; first < q0 + n_own; first += 32)
             {
-                const uint32_t ql = 32 * half + (lane >> 1);
-                const bool theirs = (finite >> ql) & 1ull;
-                done = __ballot(((lane >> 5) == half) && mine && (around > kFewPair * rows || inner < limit)) == 0;
+                const uint32_t count = min(32u, q0 + n_own - first), ql = (first + (lane >> 1)) & 63u;
+                done = __ballot(own && lane - first < count &&
+                                (around > (rows > 5 ? kFewVolume : kFewPair) * rows || inner < limit)) == 0;
                 if (!done) break;
                 const float x = __uint_as_float(from_lane(__float_as_uint(qv.x), ql)),
-                            y0 = __uint_as_float(from_lane(__float_as_uint(qv.y), ql)),
-                            z0 = __uint_as_float(from_lane(__float_as_uint(qv.z), ql));
-                const int px = (int)from_lane((uint32_t)cx, ql), py = (int)from_lane((uint32_t)cy, ql),
-                          pz = (int)from_lane((uint32_t)cz, ql);
+                            y = __uint_as_float(from_lane(__float_as_uint(qv.y), ql)),
+                            z = __uint_as_float(from_lane(__float_as_uint(qv.z), ql));
+                const int px0 = (int)from_lane((uint32_t)x0, ql), px1 = (int)from_lane((uint32_t)x1, ql),
+                          p_rows = (int)from_lane(lane - first < count ? (uint32_t)n_rows : 0u, ql);
+                Rows S = rows_from(from_lane(first_row, ql), (int)from_lane((uint32_t)ny, ql));
                 uint32_t got = 0;
 #pragma unroll 1
-                for (int r = 0; r < 9; ++r)
+                for (int r = 0; r < 9; ++r, S.next())
                 {
-                    const int y = py + r % 3 - 1, z = pz + r / 3 - 1;
+                    if (__ballot(r < p_rows) == 0) break;
                     uint32_t j = 0, e = 0;
-                    if (theirs && (uint32_t)y < (uint32_t)a1 && (uint32_t)z < (uint32_t)a2)
+                    if (r < p_rows)
                     {
-                        const uint32_t at = ((uint32_t)z * (uint32_t)a1 + (uint32_t)y) * (uint32_t)a0;
-                        j = gload(tcs, at + (uint32_t)max(px - 1, 0)) + 4u * odd;
-                        e = gload(tcs, at + (uint32_t)min(px + 1, a0 - 1) + 1u);
+                        j = gload(tcs, S.at + (uint32_t)px0) + 4u * odd;
+                        e = gload(tcs, S.at + (uint32_t)px1 + 1u);
                     }
                     for (; j < e; j += 8)
                     {
@@ -670,7 +729,7 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
 #pragma unroll
                         for (uint32_t u = 0; u < 4; ++u)
                         {
-                            const uint32_t d = min(__float_as_uint(sqdist32(x, y0, z0, p[u].x, p[u].y, p[u].z)), kNanBits);
+                            const uint32_t d = min(__float_as_uint(sqdist32(x, y, z, p[u].x, p[u].y, p[u].z)), kNanBits);
                             if (j + u < e && d <= limit)
                             {
                                 if (got < kPair)
@@ -696,7 +755,7 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
 #pragma unroll
                 for (int r = 0; r < kPerLane; ++r) prow[odd * kPerLane + r] = (uint64_t)__double_as_longlong(v[r]);
                 wave_sync();
-                write_rows(32 * half, min(32u, nq - 32 * half), kPairStride, from_lane(both, (2 * lane) & 63u));
+                write_rows(first, count, kPairStride, from_lane(both, (2 * lane) & 63u));
                 wave_sync();
             }
             if (done) return;
