@@ -660,17 +660,24 @@ bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
     return k <= kWaveMaxK && (double)k <= tuning().wave_k_max;
 }
 
-// Whether the plan chooses between the two searches once it has seen how the
-// cloud fills its box: small k of large clouds searching themselves.  A wave
-// spends most of such a query on its region, a lane per query a step per
-// candidate, and what that loses is its lanes' uneven work: it loses little
-// where points lie evenly in a volume, and a wave much where cells at the
-// grid's cap hold points by the dozen (us per call, general / wave: uniform
-// points 1 M at k = 2 482 / 521, k = 8 573 / 540; 1.5 M 605 / 743, 726 / 781;
-// 10 M 3396 / 4649, 4048 / 4855, at k = 10 4307 / 4721, k = 12 4769 / 4711; 10
-// M LiDAR points 5447 / 4999, 8001 / 5509; a scanner's rings, 4 M points, 2669 /
-// 3822, 3782 / 4232, 2 M points 1737 / 2087, 2367 / 2286).  Both are queued, one
-// finds nothing to do: about 30 us, so not for smaller clouds.
+// Whether the plan chooses between the two searches (k_plan_levels) once it
+// has seen how the cloud fills its box: small k of large clouds searching
+// themselves.  A wave spends most of such a query on its region; a lane per
+// query loses by its lanes' uneven work and by the queries that it defers.  The
+// general search takes clouds
+// - that fill a volume evenly: the probe counts no more than twice the points
+//   per cell that an even spread has;
+// - of a sheet, whose cells reach their target with points all over them
+//   (within a quarter), k <= 4 from 1 M points per neighbour on;
+// - whose points crowd, 20 in a cell on average with the cells at the grid's
+//   cap, from 400 k points per neighbour on.
+// us per call, by wave / general: uniform points 1 M at k = 2 521 / 482, k = 8
+// 540 / 573; 4 M k = 2 1838 / 1409, k = 10 1927 / 1875; 10 M 4566 / 3441, 4753 /
+// 4426, k = 12 4711 / 4769.  Rolling ground of 4 M points k = 2 1742 / 1217, k = 4
+// 1746 / 1360, k = 10 1737 / 1890, with trees on it 2144 / 1873, 2251 / 2298, 2661 /
+// 3226.  A scanner's turns over one another, 4 M points: k = 2 3620 / 2590, k = 10
+// 4069 / 3955.  LiDAR street scenes, 10 M points: 5027 / 5455, 5601 / 8396.  Both
+// are queued, one finds nothing to do: about 30 us, so not for smaller clouds.
 bool search_choice(uint32_t k, bool self, uint32_t n) { return self && k >= 2 && k <= 10 && n >= (5u << 18); }
 
 // Sort `data` into a pyramid of uniform grids (cell edge h_0 * ratio^l) and,

@@ -64,7 +64,7 @@ struct LevelTable
     Level probe;             // kNN sizing probe grid (cs, pts unused)
     uint64_t probe_G;
     float bb[8];             // bounding box of the finite data coordinates: lo xyz, hi xyz
-    unsigned long long sumsq;  // probe: sum of squared cell counts
+    unsigned long long sumsq, sumsq_clip;  // probe: sum of squared cell counts, and with crowded cells' counts clipped
     double hcap, T, h1;      // planning intermediates (grid-size floor, target occupancy, first guess)
     // kNN: queries of the general search (count[0], where the plan chooses between
     // it and the wave search) and those left after each budgeted pass

@@ -280,25 +280,32 @@ __global__ __launch_bounds__(256) void k_hist_probe(const float* __restrict__ xy
     atomicAdd(&count[cell_id(L, (double)xyz[i * 3 + 0], (double)xyz[i * 3 + 1], (double)xyz[i * 3 + 2])], 1u);
 }
 
-__global__ __launch_bounds__(256) void k_sumsq(const uint32_t* __restrict__ count, LevelTable* __restrict__ tab)
+// Sum of the counts' squares; sumsq_clip: a cell's points count as in one of
+// 8 crowded ones at most, so that a single tight cluster crowds no cloud.
+constexpr double kCrowdedCell = 20.0;  // points per cell of level 0
+__global__ __launch_bounds__(256) void k_sumsq(const uint32_t* __restrict__ count, uint32_t stride,
+                                               LevelTable* __restrict__ tab)
 {
     const uint64_t G = tab->probe_G;
-    unsigned long long* out = &tab->sumsq;
-    unsigned long long acc = 0;
+    const double edge = tab->h1 / tab->hcap;
+    const uint32_t clip = (uint32_t)fmin(1.0 + 8.0 * kCrowdedCell * edge * edge / (double)stride, 4e9);
+    unsigned long long acc = 0, acc_clip = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < G; i += (uint64_t)gridDim.x * 256)
     {
         const unsigned long long c = count[i];
         acc += c * c;
+        acc_clip += c * min(count[i], clip);
     }
-    __shared__ unsigned long long s[256];
-    s[threadIdx.x] = acc;
+    __shared__ unsigned long long s[2][256];
+    s[0][threadIdx.x] = acc, s[1][threadIdx.x] = acc_clip;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1)
     {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
+        if ((int)threadIdx.x < w)
+            s[0][threadIdx.x] += s[0][threadIdx.x + w], s[1][threadIdx.x] += s[1][threadIdx.x + w];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(out, s[0]);
+    if (threadIdx.x < 2) atomicAdd(threadIdx.x ? &tab->sumsq_clip : &tab->sumsq, s[threadIdx.x][0]);
 }
 
 // ------------------------------------------------------ grid planning ----
@@ -381,7 +388,7 @@ __global__ __launch_bounds__(256) void k_bbox_plan(const float* __restrict__ par
     plan_extent(bb, ext, emax);
     const double hcap = plan_h_for_cap(ext, p.cap);
     tab->hcap = hcap;
-    tab->sumsq = 0;
+    tab->sumsq = tab->sumsq_clip = 0;
     tab->probe_G = 0;
     tab->n_levels = 0;
     for (int l = 0; l < kMaxLevels; ++l) tab->G[l] = 0;
@@ -449,19 +456,22 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
         h = fmax(h, hcap);
         if (p.choose)
         {
-            // The general search takes clouds that fill a volume evenly (its
-            // lanes have the same work, hardly a query is deferred), with its
-            // own smaller cells, and those whose points crowd in cells at the
-            // cap (candidates by the hundred for a few neighbours, at
-            // 400 k points per neighbour); see search_choice().
-            const bool even = m1 <= 2.0 * T;
-            const bool crowded = m1 * (h / h1) * (h / h1) > 30.0 && (double)p.n >= 4e5 * (double)p.k;
+            // see search_choice()
+            const double at = m1 * (h / h1) * (h / h1);
+            const double mc = ((double)tab->sumsq_clip - (1.0 - pf) * ns) / (pf * fmax(ns, 1.0));
+            const bool even = m1 <= 2.0 * T || (at <= 1.25 * T && p.k <= 4 && (double)p.n >= 1e6 * (double)p.k);
+            const bool crowded = mc * (h / h1) * (h / h1) > kCrowdedCell && (double)p.n >= 4e5 * (double)p.k;
             if (even)
             {
                 const double Tg = fmax(0.75, fmin(p.general_occupancy * (double)p.k, p.knn_cell_points_max));
-                const double mg = 1.0 + (m1 - 1.0) * Tg / T;
-                h = h1 * cbrt(Tg / T);
-                if (mg > Tg) h *= sqrt(Tg / mg);
+                if (m1 <= 2.0 * T)
+                {
+                    const double mg = 1.0 + (m1 - 1.0) * Tg / T;
+                    h = h1 * cbrt(Tg / T);
+                    if (mg > Tg) h *= sqrt(Tg / mg);
+                }
+                else
+                    h = h1 * sqrt(Tg / m1);
                 h = fmax(h, hcap);
             }
             tab->count[0] = even || crowded ? p.n : 0;
@@ -2604,7 +2614,7 @@ hipError_t launch_probe(const float* xyz, uint32_t n, uint32_t stride, LevelTabl
     if (e != hipSuccess) return e;
     k_hist_probe<<<(ns + 255) / 256, 256, 0, s>>>(xyz, n, stride, tab, count);
     // (each block ends in one atomic on the same word: 2048 of them took 26 us)
-    k_sumsq<<<blocks_for(count_room, 256, 128), 256, 0, s>>>(count, tab);
+    k_sumsq<<<blocks_for(count_room, 256, 128), 256, 0, s>>>(count, stride, tab);
     return hipGetLastError();
 }
 

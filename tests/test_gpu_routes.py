@@ -188,3 +188,13 @@ def test_sparse_radius_time():
     1.25."""
     x = torch.from_numpy(scenes.lidar_scene(1_000_000, seed=5, extent=63.0)).cuda()
     assert _ratio(lambda: pgeof.radius_search(x, x, 0.02, 24)) < 1.25
+
+
+def test_one_cluster_time():
+    """3 M points of which a 64th stand in one tight cluster, k = 7: they alone
+    crowd no cloud, and the wave search takes it: 0.6 of the general search's
+    time.  The limit lies at 0.85."""
+    x = _uniform(3_000_000)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x[: len(x) // 64] = 0.5 + 1e-4 * torch.randn(len(x) // 64, 3, generator=g, device="cuda")
+    assert _ratio(lambda: pgeof.knn_search(x, x, 7)) < 0.85
