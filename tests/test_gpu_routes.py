@@ -198,3 +198,27 @@ def test_one_cluster_time():
     g = torch.Generator(device="cuda").manual_seed(1)
     x[: len(x) // 64] = 0.5 + 1e-4 * torch.randn(len(x) // 64, 3, generator=g, device="cuda")
     assert _ratio(lambda: pgeof.knn_search(x, x, 7)) < 0.85
+
+
+@pytest.mark.parametrize("k", [8, 20])
+def test_firing_order_time(k):
+    """2 M points stored by 64 rings, one of which scatters far: the probe that
+    sizes the grid must not see that one alone.  In firing order 2.2 (k = 20)
+    and 5.3 times (k = 8) as long as shuffled with a fixed stride; the limit
+    lies at 1.4."""
+    n, extent = 1 << 21, 92.0
+    xyz = scenes.lidar_scene(n, seed=12, extent=extent).reshape(-1, 64, 3)
+    xyz[:, 0] = scenes.uniform_cube(len(xyz), seed=2) * np.float32([extent, extent, 40.0])
+    x = torch.from_numpy(xyz.reshape(-1, 3)).cuda()
+    y = x[torch.randperm(n, generator=torch.Generator(device="cuda").manual_seed(1), device="cuda")].contiguous()
+
+    def ms(x):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        pgeof.knn_search(x, x, k)
+        torch.cuda.synchronize()
+        return time.perf_counter() - t
+
+    ratio = np.median([ms(x) / ms(y) for _ in range(8)][2:])
+    print(f"firing order over shuffled: {ratio:.2f}")
+    assert ratio < 1.4
