@@ -668,12 +668,13 @@ bool wave_path(uint32_t k, bool radius, bool self, uint32_t n)
 // - that fill a volume evenly: the probe counts no more than twice the points
 //   per cell that an even spread has;
 // - of a sheet, whose cells reach their target with points all over them
-//   (within a quarter), k <= 4 from 1 M points per neighbour on;
+//   (within a quarter), k <= 4 from 500 k points per neighbour on;
 // - whose points crowd, 20 in a cell on average with the cells at the grid's
 //   cap, from 400 k points per neighbour on.
 // us per call, by wave / general: uniform points 1 M at k = 2 521 / 482, k = 8
 // 540 / 573; 4 M k = 2 1838 / 1409, k = 10 1927 / 1875; 10 M 4566 / 3441, 4753 /
-// 4426, k = 12 4711 / 4769.  Rolling ground of 4 M points k = 2 1742 / 1217, k = 4
+// 4426, k = 12 4711 / 4769.  Rolling ground of 1.4 M points, k = 2 654 / 467, with
+// trees on it 811 / 779, k = 4 655 / 525, 846 / 937; 4 M k = 2 1742 / 1217, k = 4
 // 1746 / 1360, k = 10 1737 / 1890, with trees on it 2144 / 1873, 2251 / 2298, 2661 /
 // 3226.  A scanner's turns over one another, 4 M points: k = 2 3620 / 2590, k = 10
 // 4069 / 3955.  LiDAR street scenes, 10 M points: 5027 / 5455, 5601 / 8396.  Both

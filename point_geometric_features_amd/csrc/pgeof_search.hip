@@ -467,7 +467,7 @@ __global__ void k_plan_levels(PlanArgs p, LevelTable* __restrict__ tab)
             // see search_choice()
             const double at = m1 * (h / h1) * (h / h1);
             const double mc = ((double)tab->sumsq_clip - (1.0 - pf) * ns) / (pf * fmax(ns, 1.0));
-            const bool even = m1 <= 2.0 * T || (at <= 1.25 * T && p.k <= 4 && (double)p.n >= 1e6 * (double)p.k);
+            const bool even = m1 <= 2.0 * T || (at <= 1.25 * T && p.k <= 4 && (double)p.n >= 5e5 * (double)p.k);
             const bool crowded = mc * (h / h1) * (h / h1) > kCrowdedCell && (double)p.n >= 4e5 * (double)p.k;
             if (even)
             {
