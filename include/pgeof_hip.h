@@ -256,7 +256,13 @@ void pgeof_server_destroy(pgeof_server* server);
  * (wave-shared LDS staging of cell rows: 0 never (default: each lane streams
  * its rows' candidates from L2), 1 radius search and, for k >= 32, the
  * budgeted kNN pass, 2 radius search and the budgeted kNN pass at any k), "fuse_multiscale" (pgeof_radius_multiscale_device: 1 the
- * features in the search kernel, 0 in a CSR kernel after it).
+ * features in the search kernel, 0 in a CSR kernel after it), "wave_k_max"
+ * (largest k, or radius cap, of the search with one wave per query, at most
+ * 108; 0: never).  That search takes kNN of k up to it and radius searches of
+ * caps 22 up to it, but for k = 1 of clouds of 2^16 points and more that search
+ * themselves, and for k = 2 to 10 of ones of 1.3 M points and more whose
+ * grid plan finds the other search faster; it reads none of "lds_budget",
+ * "near_first", "budget_*", "heap_tail" and "staging".
  * Knobs change speed only, never results. Values must be finite and >= 0. */
 int pgeof_set_tuning(const char* key, double value);
 double pgeof_get_tuning(const char* key);

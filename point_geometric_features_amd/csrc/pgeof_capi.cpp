@@ -1746,7 +1746,9 @@ int pgeof_autotune(const char* workload, const float* xyz, int64_t n, uint32_t k
     if (family == kFamKnn)
     {
         // (the wave-per-query search has no heaps and stages no rows)
-        const bool wave = k <= kWaveMaxK && (double)k <= base.wave_k_max;
+        t_snap = &base;
+        const bool wave = wave_path(k, false, true, (uint32_t)n) && !search_choice(k, true, (uint32_t)n);
+        t_snap = nullptr;
         for (double cpp : {4.0, 8.0, 16.0})
             for (double occ : {0.25, 0.35, 0.5})
                 for (double lds : {65536.0, 32768.0})
@@ -1763,10 +1765,16 @@ int pgeof_autotune(const char* workload, const float* xyz, int64_t n, uint32_t k
     }
     else
     {
+        // (features after the search: the search may be the wave-per-query one,
+        // which stages no rows)
+        t_snap = &base;
+        const bool wave = wave_path(k, true, true, (uint32_t)n);
+        t_snap = nullptr;
         for (double rcf : {0.35, 0.5, 0.7, 1.0})
             for (double fu : {0.0, 1.0})
                 for (double st : {0.0, 1.0})
                 {
+                    if (wave && fu == 0.0 && st != 0.0) continue;
                     Tuning t = base;
                     t.radius_cell_factor = rcf;
                     t.fuse_multiscale = fu;
