@@ -15,7 +15,7 @@
 // per lane.
 //
 // What bounds it: instruction issue and the latency of the few dependent
-// loads per region, at 12 waves per CU (registers; the LDS rows allow 13):
+// loads per region, at 12 or 13 waves per CU (registers; LDS rows):
 // 10 M LiDAR points at k = 20 take about 200 vector instructions per query
 // (k_search, a lane per query with a heap, about 430, its lanes waiting for
 // each other: 3 times the candidate steps and 3.5 times the insertions of a
@@ -126,12 +126,6 @@ __device__ __forceinline__ void order2(double& a, double& b)
     asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
     a = lo;
     b = hi;
-}
-
-// a key as a double
-__device__ __forceinline__ double key_bits(uint32_t d, uint32_t id)
-{
-    return __longlong_as_double((long long)(((uint64_t)d << 32) | id));
 }
 
 template <int CTRL>
@@ -425,13 +419,15 @@ __device__ __forceinline__ uint32_t work_block(uint32_t b, uint32_t nb)
 }
 
 // G: lanes that sort one query's row of kPerLane * G kept candidates.
-// Three waves per SIMD (168 registers): nothing spills but scalars, and the
-// LDS rows allow 13 waves per CU at most.  With four (128 registers, 5 to 9 of
-// them spilled for G <= 2): 10 M LiDAR points, k = 20, fused 7.75 ms instead
-// of 7.65, 300 k 486 us instead of 435, 1 M at k = 8 719 instead of 654; 1 M
-// uniform points at k = 20 602 instead of 616.
-template <int MODE, int G>
-__global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
+// WAVES per SIMD: with three (168 registers) nothing spills but scalars (up to
+// three vector registers of the radius modes).  With four (128 registers) four
+// or five spill, which k = 9 to 27 repay where the launch keeps four waves on
+// every SIMD (us per call, fused, three / four: 10 M LiDAR points at k = 20, mean
+// of eight clouds, 7650 / 7310; 1 M 946 / 917; 1 M uniform points 717 / 685; 300 k
+// 291 / 280; 10 k 75.8 / 79.4); k <= 8 is slower with four (1 M LiDAR points at k =
+// 8 762 / 784), larger rows do not fit.
+template <int MODE, int G, int WAVES>
+__global__ __launch_bounds__(64, WAVES) void k_wave_search(WaveArgs a)
 {
     constexpr bool RADIUS = MODE == kModeRadius || MODE == kModeRadiusCsr;
     if (!RADIUS && a.other && *a.other) return;
@@ -1048,7 +1044,8 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
                             {
                                 const uint32_t d = min(__float_as_uint(sqdist32(qxf, qyf, qzf, p[u].x, p[u].y, p[u].z)), kNanBits);
                                 const uint32_t id = __float_as_uint(p[u].w);
-                                const bool in = (f0 + u * 64u + lane < tot) & (key_bits(d, id) <= key_bits(tau, tie));
+                                bool in = (f0 + u * 64u + lane < tot) & (d <= tau);
+                                if (tie != 0xFFFFFFFFu) in &= (d < tau) | (id <= tie);
                                 const uint64_t m = __ballot(in);
                                 if (in) buf[n_buf + lanes_below(m)] = ((uint64_t)d << 32) | id;
                                 n_buf = uniform(n_buf + (uint32_t)__popcll(m));
@@ -1155,23 +1152,31 @@ __global__ __launch_bounds__(64, 3) void k_wave_search(WaveArgs a)
     }
 }
 
+template <int G, int WAVES>
+hipError_t launch_wave_w(int mode, uint32_t nb, const WaveArgs& a, hipStream_t s)
+{
+    if (mode == kModeKnn)
+        k_wave_search<kModeKnn, G, WAVES><<<nb, 64, 0, s>>>(a);
+    else if (mode == kModeKnnFeat)
+        k_wave_search<kModeKnnFeat, G, WAVES><<<nb, 64, 0, s>>>(a);
+    else if constexpr (G >= 4)
+    {
+        if (mode == kModeRadius)
+            k_wave_search<kModeRadius, G, WAVES><<<nb, 64, 0, s>>>(a);
+        else
+            k_wave_search<kModeRadiusCsr, G, WAVES><<<nb, 64, 0, s>>>(a);
+    }
+    return hipGetLastError();
+}
+
 template <int G>
 hipError_t launch_wave_g(int mode, const WaveArgs& a, hipStream_t s)
 {
     const bool radius = mode == kModeRadius || mode == kModeRadiusCsr;
     const uint32_t nb = radius ? (a.n_query + 63) / 64 * (64 / a.q_per_wave) : (a.n_query + a.q_per_wave - 1) / a.q_per_wave;
-    if (mode == kModeKnn)
-        k_wave_search<kModeKnn, G><<<nb, 64, 0, s>>>(a);
-    else if (mode == kModeKnnFeat)
-        k_wave_search<kModeKnnFeat, G><<<nb, 64, 0, s>>>(a);
-    else if constexpr (G >= 4)
-    {
-        if (mode == kModeRadius)
-            k_wave_search<kModeRadius, G><<<nb, 64, 0, s>>>(a);
-        else
-            k_wave_search<kModeRadiusCsr, G><<<nb, 64, 0, s>>>(a);
-    }
-    return hipGetLastError();
+    if constexpr (G == 2)
+        if (nb > 4u * 1024u) return launch_wave_w<G, 4>(mode, nb, a, s);  // (1024 SIMDs)
+    return launch_wave_w<G, 3>(mode, nb, a, s);
 }
 
 }  // namespace
