@@ -685,7 +685,7 @@ bool search_choice(uint32_t k, bool self, uint32_t n) { return self && k >= 2 &&
 // when query != data, sort the queries into level 0.  kNN sizes h_0 from the
 // target occupancy (k used for sizing); radius searches use one level with
 // cells of radius_cell_factor * radius.  The sizes are planned on the device
-// (k_plan_probe, k_plan_levels): every launch is queued without a read-back,
+// (k_bbox_plan, k_plan_levels): every launch is queued without a read-back,
 // the kernels take their grid from the level table and the launches are
 // sized for the largest grid the workspace allows.
 int build_grid(const float* data, uint32_t n, const float* query, uint32_t m, uint32_t k, float radius, bool is_radius,

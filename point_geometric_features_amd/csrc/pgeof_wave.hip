@@ -20,7 +20,7 @@
 // (k_search, a lane per query with a heap, about 430, its lanes waiting for
 // each other: 3 times the candidate steps and 3.5 times the insertions of a
 // lane).  Search kernels per call, k_search -> this one: 10 M at k = 20 9.8 ->
-// 6.0 ms, 4 M at k = 50 12.5 -> 3.7 ms, 1 M uniform points at k = 50 2.6 ->
+// 5.9 ms, 4 M at k = 50 12.5 -> 3.7 ms, 1 M uniform points at k = 50 2.6 ->
 // 0.65 ms, 1 M at k = 100 7.1 -> 2.1 ms, 100 k at k = 20 1.8 -> 0.2 ms (there
 // single sparse queries held a lane for thousands of steps).
 #include <type_traits>
@@ -370,8 +370,6 @@ struct Candidates
 };
 
 // --------------------------------------------------------- the kernel ----
-// Candidates of a cell's 3x3x3 cube kept in registers, in groups of 64 (one
-// per lane); larger cubes are streamed instead.
 // A level of the table, read with scalar loads (the table was written by
 // earlier kernels and does not change during this one).
 #define PGEOF_CONST __attribute__((address_space(4)))
@@ -380,6 +378,8 @@ __device__ __forceinline__ const PGEOF_CONST Level* scalar_level(const LevelTabl
     return (const PGEOF_CONST Level*)(tab->lv + l);
 }
 
+// Candidates of a cell's 3x3x3 cube kept in registers, in groups of 64 (one
+// per lane); larger cubes are streamed instead.
 template <int G>
 constexpr uint32_t kGroupsOf = G <= 2 ? 6 : 12;
 // Streamed candidates collected in LDS before the farthest are dropped.
