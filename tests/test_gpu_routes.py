@@ -222,3 +222,39 @@ def test_firing_order_time(k):
     ratio = np.median([ms(x) / ms(y) for _ in range(8)][2:])
     print(f"firing order over shuffled: {ratio:.2f}")
     assert ratio < 1.4
+
+
+def test_choice_in_a_graph():
+    """The choice is the plan's, on the device: one captured call serves clouds
+    that go to either search, swapped between replays."""
+    n, k = 5 << 18, 5
+    clouds = [_uniform(n), torch.from_numpy(scenes.lidar_scene(n, seed=11, extent=72.0)).cuda()]
+    x = clouds[0].clone()
+    out = [torch.empty(n * k, dtype=torch.int32, device="cuda"), torch.empty(n + 1, dtype=torch.int32, device="cuda"),
+           torch.empty(n, 11, device="cuda")]
+    ws = torch.empty(capi.knn_workspace_size(n, n, k), dtype=torch.uint8, device="cuda")
+    want = []
+    for cloud in clouds:
+        x.copy_(cloud)
+        capi.knn_features_device(x, k, *out, workspace=ws)
+        want.append([o.clone() for o in out])
+    with _General():
+        capi.knn_features_device(x, k, *out, workspace=ws)
+    assert torch.equal(out[0], want[1][0]) and torch.equal(out[2], want[1][2])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        capi.knn_features_device(x, k, *out, workspace=ws, stream=side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        capi.knn_features_device(x, k, *out, workspace=ws, stream=torch.cuda.current_stream())
+    for i in (0, 1, 1, 0, 1, 0):
+        for o in out:
+            o.fill_(-3)
+        x.copy_(clouds[i])
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, w in zip(out, want[i]):
+            assert torch.equal(o, w)
