@@ -852,6 +852,12 @@ int run_search(int mode, const float* data, uint32_t n, const float* query, uint
         // wave, 145 with 1).  For radius searches a power of two: the waves
         // of 64 queries share them where they are sparse.
         b.q_per_wave = std::max<uint32_t>(1, std::min<uint32_t>(64u, std::max(std::min<uint32_t>(32u, m / 2048), m / 32768)));
+        // A little over 3072 waves (three per SIMD) the last ones would wait for a
+        // place: a query or two more for each instead (100 k uniform points, k =
+        // 20: 154 us per call with 32, 136 with 33; LiDAR 268, 271).  Six more
+        // cost LiDAR scenes what they save elsewhere (115 k: 267 -> 285; 160 ->
+        // 145).
+        if (m > 3072u * 32u && m <= 3072u * 34u) b.q_per_wave = (m + 3071u) / 3072u;
         if (is_radius)
             while (b.q_per_wave & (b.q_per_wave - 1)) b.q_per_wave &= b.q_per_wave - 1;
         b.other = choose ? &w.tab->count[0] : nullptr;

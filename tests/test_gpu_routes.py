@@ -258,3 +258,19 @@ def test_choice_in_a_graph():
         torch.cuda.synchronize()
         for o, w in zip(out, want[i]):
             assert torch.equal(o, w)
+
+
+@pytest.mark.parametrize("n", [98_304, 98_305, 101_377, 104_448, 104_449])
+@pytest.mark.parametrize("k", [8, 20, 60])
+def test_queries_per_wave(n, k):
+    """Around the sizes where a wave takes 32, 33 or 34 queries."""
+    xyz = scenes.lidar_scene(n, seed=7, extent=20.0)
+    x = torch.from_numpy(xyz).cuda()
+    gi, gd = pgeof.knn_search(x, x, k)
+    with _General():
+        wi, wd = pgeof.knn_search(x, x, k)
+    assert torch.equal(gi, wi) and torch.equal(gd, wd)
+    ri, rd = pgeof.radius_search(x, x, 0.3, k + 20)
+    with _General():
+        wi, wd = pgeof.radius_search(x, x, 0.3, k + 20)
+    assert torch.equal(ri, wi) and torch.equal(rd, wd)
